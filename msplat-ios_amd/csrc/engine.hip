@@ -101,9 +101,9 @@ struct Engine {
     int64_t dens_rows = 0;  // rows dens_ws and dens_keep are sized for
     DevBuf pair_counter;
     DevBuf rgba;  // RGBA8 staging of msplat_hip_image_to_rgba8
-    // mesh extraction: TSDF view records and pixel masks, marching-cubes case
+    // mesh extraction: TSDF view records and block maxima, marching-cubes case
     // bytes, and the per-chunk counts / scanned offsets of the two compactions
-    DevBuf tsdf_views, tsdf_masks, mc_cases, chunk_cnt, chunk_off;
+    DevBuf tsdf_views, tsdf_blocks, mc_cases, chunk_cnt, chunk_off;
     // state of the most recent forward
     int n = 0, W = 0, H = 0, tiles_x = 0, tiles_y = 0, K3 = 0;
     int64_t num_isect = 0;
@@ -780,7 +780,7 @@ void msplat_hip_cleanup(void) {
                      &E.final_idx, &E.out_depth, &E.out_normal, &E.out_alpha, &E.out_median, &E.out_dist,
                      &E.dL_dimg, &E.gm1, &E.gs1, &E.gs12, &E.partials, &E.loss, &E.dmeans, &E.dscales,
                      &E.dquats, &E.dmean2d, &E.dfdc, &E.dfrest, &E.dens_flags, &E.dens_scan, &E.dens_keep, &E.dens_ws, &E.deep_list, &E.deep_pos, &E.deep_tb, &E.deep_cnt, &E.log_table, &E.log_ctr, &E.pair_counter,
-                     &E.rgba, &E.tsdf_views, &E.tsdf_masks, &E.mc_cases, &E.chunk_cnt, &E.chunk_off};
+                     &E.rgba, &E.tsdf_views, &E.tsdf_blocks, &E.mc_cases, &E.chunk_cnt, &E.chunk_off};
     for (DevBuf *b : all) {
         if (b->p) (void)hipFree(b->p);
         *b = DevBuf{};
@@ -965,32 +965,34 @@ int msplat_hip_tsdf_integrate(float *grid, int dx, int dy, int dz, const float o
         }
     if (num_views == 0) return MSPLAT_OK;
     Engine &E = g_eng;
-    // each view's pass mask, then the fold
+    // each view's block maxima, then the fold
     std::vector<mskern::TsdfViewDev> dv((size_t)num_views);
-    size_t words = 0;
-    int64_t max_segs = 0;
+    size_t blocks = 0;
+    int64_t max_tasks = 0;
     for (int k = 0; k < num_views; ++k) {
+        const int bw = (views[k].width - 1) / mskern::kTsdfBlock + 1, bh = (views[k].height - 1) / mskern::kTsdfBlock + 1;
         dv[k].v = views[k];
-        dv[k].words_per_row = mskern::tsdf_mask_words(views[k].width);
-        words += (size_t)dv[k].words_per_row * views[k].height;
-        max_segs = std::max<int64_t>(max_segs, (int64_t)((views[k].width + 63) / 64) * views[k].height);
+        dv[k].blk_w = bw;
+        blocks += (size_t)bw * bh;
+        max_tasks = std::max<int64_t>(max_tasks, mskern::tsdf_block_tasks(views[k].width, views[k].height));
     }
-    if (max_segs > (int64_t)INT_MAX) {
+    if (max_tasks > (int64_t)INT_MAX) {
         set_err("TSDF view too large");
         return MSPLAT_E_ARG;
     }
-    CHECK(ensure(E.tsdf_masks, words * 4));
+    CHECK(ensure(E.tsdf_blocks, blocks * 4));
     size_t off = 0;
     for (auto &d : dv) {
-        d.mask = P<uint32_t>(E.tsdf_masks) + off;
-        off += (size_t)d.words_per_row * d.v.height;
+        d.blk = P<float>(E.tsdf_blocks) + off;
+        off += (size_t)d.blk_w * ((d.v.height - 1) / mskern::kTsdfBlock + 1);
     }
     const size_t bytes = dv.size() * sizeof(mskern::TsdfViewDev);
     CHECK(ensure(E.tsdf_views, bytes));
     HIPC(hipMemcpyAsync(E.tsdf_views.p, dv.data(), bytes, hipMemcpyHostToDevice, E.stream));
     const auto *vdev = P<mskern::TsdfViewDev>(E.tsdf_views);
-    mskern::launch_tsdf_masks(E.stream, vdev, num_views, max_segs, alpha_thresh);
-    mskern::launch_tsdf_integrate(E.stream, grid, dx, dy, dz, origin, voxel_size, vdev, num_views, trunc_dist);
+    mskern::launch_tsdf_blocks(E.stream, vdev, num_views, max_tasks, alpha_thresh);
+    mskern::launch_tsdf_integrate(E.stream, grid, dx, dy, dz, origin, voxel_size, vdev, num_views, trunc_dist,
+                                  alpha_thresh);
     HIPC(hipGetLastError());
     // the view records are rewritten by the next call
     HIPC(hipStreamSynchronize(E.stream));

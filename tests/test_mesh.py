@@ -350,6 +350,58 @@ def test_gpu_tsdf_matches_oracle(orc, eng):
     assert np.array_equal(got.view(np.uint32), grid.view(np.uint32))
 
 
+# (grid, voxel size, views, image, eye distance): one voxel; bricks cut at
+# every face; more views than one test round (32); voxels tens of pixels wide
+# (a brick's footprint spans thousands of blocks); cameras inside the grid
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,vs,n_views,hw,dist", [
+    ((1, 1, 1), 0.1, 3, (64, 70), 1.0),
+    ((5, 9, 17), 0.02, 33, (33, 47), 1.0),
+    ((21, 30, 41), 0.02, 65, (120, 161), 1.0),
+    ((6, 10, 9), 0.15, 5, (900, 1100), 1.2),
+    ((24, 24, 24), 0.05, 12, (97, 130), 0.45),
+])
+def test_gpu_tsdf_brick_test_drops_nothing(dims, vs, n_views, hw, dist, orc, eng):
+    """The fold skips a view for a whole brick of voxels when its block
+    maxima show that no voxel can change; the grid must still be the golden
+    model's bit for bit."""
+    from msplat import _engine as E
+    rng = np.random.default_rng(sum(dims) + n_views)
+    dz, dy, dx = dims
+    H, W = hw
+    origin = (-0.5 * vs * np.array([dx, dy, dz])).astype(np.float32)
+    grid = np.zeros((dz, dy, dx, 2), np.float32)
+    dev = E.DeviceArray.from_numpy(grid)
+    radius = 0.3 * vs * max(dims)
+    views, keep = [], []
+    for k in range(n_views):
+        eye = dist * _unit(rng.normal(size=3))
+        fwd = _unit(rng.normal(scale=0.1, size=3) - eye)
+        right = _unit(np.cross(fwd, rng.normal(size=3)))
+        vm = np.eye(4)
+        vm[:3, :3] = np.stack([right, np.cross(fwd, right), fwd])
+        vm[:3, 3] = -vm[:3, :3] @ eye
+        vm = vm.astype(np.float32)
+        fx, fy, cx, cy = 0.9 * W, 1.1 * W, W / 2 - 3.3, H / 2 + 1.7
+        # the depth of a ball, background elsewhere, and a few bad pixels
+        u, v = np.meshgrid((np.arange(W) + 0.5 - cx) / fx, (np.arange(H) + 0.5 - cy) / fy)
+        d = np.stack([u, v, np.ones_like(u)], -1) @ vm[:3, :3].astype(np.float64)
+        a, b, c = (d * d).sum(-1), 2 * d @ eye, eye @ eye - radius * radius
+        disc = b * b - 4 * a * c
+        depth = np.where(disc >= 0, (-b - np.sqrt(np.maximum(disc, 0))) / (2 * a), 0.0)
+        depth = (depth + rng.normal(scale=0.2 * vs, size=depth.shape)).astype(np.float32)
+        bad = rng.uniform(size=depth.shape)
+        depth[bad < 0.01] = np.nan
+        depth[bad > 0.99] = np.inf
+        alpha = np.where(disc >= 0, rng.uniform(0.4, 1.0, depth.shape), 0.0).astype(np.float32)
+        orc.tsdf_integrate(grid, origin, vs, vm, fx, fy, cx, cy, depth, alpha, 4 * vs, 0.5)
+        keep += [E.DeviceArray.from_numpy(depth), E.DeviceArray.from_numpy(alpha)]
+        views.append((vm, fx, fy, cx, cy, keep[-2], keep[-1]))
+    E.tsdf_integrate(dev, origin, vs, views, 4 * vs, 0.5)
+    assert np.array_equal(dev.numpy().view(np.uint32), grid.view(np.uint32))
+    assert (grid[..., 1] > 0).any()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("hw", [(37, 53), (64, 64), (1, 5000)])
 def test_gpu_unprojection_matches_oracle(orc, eng, hw):
