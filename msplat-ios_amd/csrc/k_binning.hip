@@ -19,8 +19,8 @@
 //      per tile, with no global atomic and no second count pass;
 //   3. k_sort_super: each super-tile counts the entries of its 16 tiles
 //      (the tile histogram, no atomics: a super-tile owns its tiles) and
-//      sorts its keys in LDS (bitonic, up to 4096 keys), larger lists in
-//      4096-key runs merged by k_merge_path; an exclusive scan of the tile
+//      sorts its keys in LDS (RunSort, up to 16384 keys), larger lists in
+//      16384-key runs merged by k_merge_path; an exclusive scan of the tile
 //      counts gives the tile offsets (the layout of the id list the
 //      rasterizers read);
 //   4. k_emit_tiles: each super-tile's sorted list is filtered, in order,
@@ -31,23 +31,21 @@
 
 namespace {
 
-constexpr int kSortThreads = 256;
-constexpr int kChunk = 4096;  // keys per LDS sort (32 KB of u64)
-// Lists longer than this are sorted, counted and emitted chunk-parallel
-// (their chunk sorts would otherwise hold one workgroup for longer than the
-// rest of the pass); shorter ones stay within their super-tile's workgroup.
-constexpr int kHuge = 4 * kChunk;
-constexpr int kSuper = 4;     // tiles per super-tile side
-static_assert(kHuge == mskern::kSuperHugeList && kChunk == mskern::kSuperSortChunk && kSuper == mskern::kSuperTile,
+constexpr int kChunk = 4096;   // keys per counting and emission unit of a huge list
+constexpr int kRun = 16384;    // keys one workgroup sorts in LDS (128 KB of u64)
+constexpr int kSuper = 4;      // tiles per super-tile side
+constexpr int kTiles = kSuper * kSuper;
+static_assert(kRun == mskern::kSuperSortRun && kChunk == mskern::kSuperChunk && kSuper == mskern::kSuperTile &&
+                  kRun % kChunk == 0,
               "the host sizes the binning buffers with these");
 
-// The merge passes (k_merge_path) take a list of cnt > kChunk keys through
-// merge_passes(cnt) passes (L = kChunk, 2 kChunk, ... below cnt), pass p
+// The merge passes (k_merge_path) take a list of cnt > kRun keys through
+// merge_passes(cnt) passes (L = kRun, 2 kRun, ... below cnt), pass p
 // reading the key buffer for even p and writing the second buffer, and the
 // reverse; merged_keys names where the list ends.
 __host__ __device__ __forceinline__ int merge_passes(int cnt) {
     int p = 0;
-    for (int64_t L = kChunk; L < cnt; L <<= 1) ++p;
+    for (int64_t L = kRun; L < cnt; L <<= 1) ++p;
     return p;
 }
 __device__ __forceinline__ const unsigned long long *merged_keys(int cnt, const unsigned long long *keys,
@@ -375,7 +373,7 @@ __device__ __forceinline__ int sort_slot(int i) { return i ^ ((i >> 3) & 31); }
 template <int M>
 __device__ __forceinline__ void bitonic_pass(unsigned long long *s, int n, int k, int lo) {
     const int groups = n >> M;
-    for (int g = threadIdx.x; g < groups; g += kSortThreads) {
+    for (int g = threadIdx.x; g < groups; g += blockDim.x) {
         const int base = ((g & ~(lo - 1)) << M) | (g & (lo - 1));
         unsigned long long v[1 << M];
 #pragma unroll
@@ -397,15 +395,15 @@ __device__ __forceinline__ void bitonic_pass(unsigned long long *s, int n, int k
     }
 }
 
-// Ascending bitonic sort of `cnt` (2..kChunk) keys in LDS (element i in
-// slot sort_slot(i)), padded to a power of two with all-ones keys: the
+// Ascending bitonic sort of the cnt (2..kRun) keys in the slots
+// sort_slot(0..cnt-1), padded to a power of two with all-ones keys: the
 // stages of each merge go three at a time through registers
 // (bitonic_pass), so a 2048-key sort takes 24 barriers instead of 66.
 // Block-uniform control flow.
-__device__ void lds_bitonic(unsigned long long *s, const unsigned long long *src, int cnt) {
+__device__ void lds_bitonic(unsigned long long *s, int cnt) {
     int n = 2;
     while (n < cnt) n <<= 1;
-    for (int i = threadIdx.x; i < n; i += kSortThreads) s[sort_slot(i)] = i < cnt ? src[i] : ~0ull;
+    for (int i = cnt + (int)threadIdx.x; i < n; i += blockDim.x) s[sort_slot(i)] = ~0ull;
     __syncthreads();
     for (int k = 2; k <= n; k <<= 1) {
         for (int j = k >> 1; j > 0;) {
@@ -424,85 +422,243 @@ __device__ void lds_bitonic(unsigned long long *s, const unsigned long long *src
     }
 }
 
-// The tile counts of a super-tile's entries keys[0, cnt): each entry covers
-// the tiles of its rectangle inside the super-tile; s_tc[16] (zeroed by the
-// caller) receives the sums.  Block-uniform.
+// Sort of up to CAP keys by one workgroup of THREADS threads, CAP / THREADS
+// keys per thread in registers.  The keys of a list are distinct and spread
+// over its depth range, so one bucket pass nearly sorts them: the position
+// of a key in [min, max] gives its bucket (a monotone map), an LDS counter
+// its place in it, a block scan of the counters the buckets' starts, and a
+// key's final place is its bucket's start plus the smaller keys in the
+// bucket -- a few, counted directly.  Seven barriers whatever the length,
+// where the bitonic network of 4096 keys takes 30.  When a bucket holds more
+// than kMaxBucket keys (depths that crowd together, for which counting
+// directly would be quadratic) the buckets are drawn again, in proportion to
+// the keys: the rank a key is expected at, interpolated linearly in its
+// first bucket, gives its new one.  Lists that crowd even then go through
+// the bitonic network.
+// Bound by LDS latency and the barriers.  Against the bitonic network (256
+// threads, 4096-key runs, longer lists merged): the 294 lists of up to ~6k
+// keys of a 1297 x 840 frame of 500k splats 63 + 8 -> 25 us, the 24 lists of
+// ~5k of a 324 x 210 frame 79 + 8 -> 22 us, the 4346 lists (1.7k on average)
+// of 5187 x 3361 with 3M splats 186 + 9 -> 109 us.
+constexpr int kMaxBucket = 48;
+template <int CAP, int THREADS>
+struct RunSort {
+    // 16 KB of counters at most: 128 KB of keys leave no more
+    static constexpr int kBuckets = CAP / 2 < 4096 ? CAP / 2 : 4096;
+    static constexpr int K = CAP / THREADS, NW = THREADS / 64, BPT = kBuckets / THREADS;
+    struct Lds {
+        unsigned long long keys[CAP];
+        int bucket[kBuckets];
+        unsigned long long mm[2 * NW];
+        int part[NW];
+        int tc[kTiles];
+    };
+    unsigned long long k[K];  // the thread's keys, j * THREADS + threadIdx.x
+
+    __device__ __forceinline__ void load(const unsigned long long *__restrict__ src, int cnt) {
+#pragma unroll
+        for (int j = 0; j < K; ++j) {
+            const int i = j * THREADS + (int)threadIdx.x;
+            k[j] = i < cnt ? src[i] : 0ull;
+        }
+    }
+
+    // Sorts the loaded keys (cnt >= 2 of them) into dst[0, cnt), which may be
+    // where they came from.
+    __device__ __forceinline__ void sort(Lds &L, unsigned long long *__restrict__ dst, int cnt) {
+        const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+        unsigned long long lo = ~0ull, hi = 0ull;
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            if (j * THREADS + tid < cnt) {
+                lo = k[j] < lo ? k[j] : lo;
+                hi = k[j] > hi ? k[j] : hi;
+            }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            const unsigned long long a = __shfl_xor(lo, d, 64), b = __shfl_xor(hi, d, 64);
+            lo = a < lo ? a : lo;
+            hi = b > hi ? b : hi;
+        }
+        if (lane == 0) {
+            L.mm[2 * wave] = lo;
+            L.mm[2 * wave + 1] = hi;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            lo = L.mm[2 * w] < lo ? L.mm[2 * w] : lo;
+            hi = L.mm[2 * w + 1] > hi ? L.mm[2 * w + 1] : hi;
+        }
+        const unsigned long long range = hi - lo;
+        const int sh = max(0, 32 - __builtin_clzll(range | 1ull));
+        // the conversion and the product are monotone, as every step of the
+        // maps below
+        const float scale = (float)kBuckets / ((float)(unsigned)(range >> sh) + 1.0f);
+        const auto place = [&](unsigned long long key) { return (float)(unsigned)((key - lo) >> sh) * scale; };
+        const float per_rank = (float)kBuckets / (float)cnt;
+        int br[K];  // bucket << 16 | arrival order in it (below 2^14)
+        bool crowded = false;
+        for (int round = 0; round < 2; ++round) {
+            if (round == 1) {
+#pragma unroll
+                for (int j = 0; j < K; ++j)
+                    if (j * THREADS + tid < cnt) {
+                        const int b = br[j] >> 16;
+                        const float f = __builtin_fminf(place(k[j]) - (float)b, 1.0f);
+                        const int b0 = L.bucket[b], b1 = b + 1 < kBuckets ? L.bucket[b + 1] : cnt;
+                        const float rank = __builtin_fminf((float)b0 + f * (float)(b1 - b0), (float)b1);
+                        br[j] = min(kBuckets - 1, (int)(rank * per_rank)) << 16;
+                    }
+                __syncthreads();
+            } else {
+#pragma unroll
+                for (int j = 0; j < K; ++j) br[j] = min(kBuckets - 1, (int)place(k[j])) << 16;
+            }
+#pragma unroll
+            for (int q = 0; q < BPT; ++q) L.bucket[q * THREADS + tid] = 0;
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if (j * THREADS + tid < cnt) br[j] |= atomicAdd(&L.bucket[br[j] >> 16], 1);
+            __syncthreads();
+            // counts -> starts; BPT consecutive buckets per thread
+            int c[BPT], sum = 0;
+            bool many = false;
+#pragma unroll
+            for (int q = 0; q < BPT; ++q) {
+                c[q] = L.bucket[BPT * tid + q];
+                many |= c[q] > kMaxBucket;
+                sum += c[q];
+            }
+            int incl = sum;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(incl, d, 64);
+                if (lane >= d) incl += o;
+            }
+            if (lane == 63) L.part[wave] = incl;
+            crowded = __syncthreads_or(many);
+            int run = incl - sum;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) run += w < wave ? L.part[w] : 0;
+#pragma unroll
+            for (int q = 0; q < BPT; ++q) {
+                L.bucket[BPT * tid + q] = run;
+                run += c[q];
+            }
+            __syncthreads();
+            if (!crowded) break;
+        }
+        if (crowded) {
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if (j * THREADS + tid < cnt) L.keys[sort_slot(j * THREADS + tid)] = k[j];
+            lds_bitonic(L.keys, cnt);
+            for (int i = tid; i < cnt; i += THREADS) dst[i] = L.keys[sort_slot(i)];
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            if (j * THREADS + tid < cnt) L.keys[L.bucket[br[j] >> 16] + (br[j] & 0xffff)] = k[j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            if (j * THREADS + tid < cnt) {
+                const int b = br[j] >> 16;
+                const int b0 = L.bucket[b], b1 = b + 1 < kBuckets ? L.bucket[b + 1] : cnt;
+                int r = b0;
+                for (int e = b0; e < b1; ++e) r += L.keys[e] < k[j] ? 1 : 0;
+                br[j] = r;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            if (j * THREADS + tid < cnt) L.keys[br[j]] = k[j];
+        __syncthreads();
+        for (int i = tid; i < cnt; i += THREADS) dst[i] = L.keys[i];
+    }
+};
+
+// The local rectangle (x0, x1, y0, y1, half-open, inside the super-tile at
+// tile (stx, sty)) of a key.
 template <bool PACKED>
-__device__ __forceinline__ void count_tiles(const unsigned long long *__restrict__ keys, int cnt, int stx, int sty,
-                                            const uint2 *__restrict__ rect, int *s_tc) {
-    int tc[kSuper * kSuper];
-#pragma unroll
-    for (int q = 0; q < kSuper * kSuper; ++q) tc[q] = 0;
-    for (int e = threadIdx.x; e < cnt; e += kSortThreads) {
-        int rx0, rx1, ry0, ry1;
-        if constexpr (PACKED) {
-            const int4 lr = unpack_rect((uint32_t)keys[e] & 0xffu);
-            rx0 = lr.x, rx1 = lr.y, ry0 = lr.z, ry1 = lr.w;
-        } else {
-            const uint2 r = rect[(uint32_t)(keys[e] & 0xffffffffull)];
-            rx0 = max((int)(r.x & 0xffff) - stx, 0), rx1 = min((int)(r.y & 0xffff) - stx, kSuper);
-            ry0 = max((int)(r.x >> 16) - sty, 0), ry1 = min((int)(r.y >> 16) - sty, kSuper);
-        }
-#pragma unroll
-        for (int q = 0; q < kSuper * kSuper; ++q) {
-            const int lx = q % kSuper, ly = q / kSuper;
-            tc[q] += (lx >= rx0 && lx < rx1 && ly >= ry0 && ly < ry1) ? 1 : 0;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < kSuper * kSuper; ++q) {
-        int v = tc[q];
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-        if ((threadIdx.x & 63) == 0 && v) atomicAdd(&s_tc[q], v);
-    }
-    __syncthreads();
+__device__ __forceinline__ int4 key_rect(unsigned long long key, int stx, int sty, const uint2 *__restrict__ rect) {
+    if constexpr (PACKED) return unpack_rect((uint32_t)key & 0xffu);
+    const uint2 r = rect[(uint32_t)(key & 0xffffffffull)];
+    return make_int4(max((int)(r.x & 0xffff) - stx, 0), min((int)(r.y & 0xffff) - stx, kSuper),
+                     max((int)(r.x >> 16) - sty, 0), min((int)(r.y >> 16) - sty, kSuper));
 }
 
-// Counts the entries of the super-tile's 16 tiles into tile_counts, then
-// sorts the super-tile list in place: up to kChunk keys in one LDS sort,
-// up to huge_th in kChunk runs queued on big_list for the merge passes.
-// Longer lists are only queued, on big_list and huge_list (their tile counts
-// zeroed): k_sort_chunks sorts their runs on many workgroups, and after the
-// merge k_count_chunks / k_emit_chunks count and emit them chunk by chunk.
-// huge_th is kHuge, or kChunk when the frame's long lists go chunk-parallel
-// (bin_chunk_parallel: some list exceeds kHuge): every list above kChunk
-// then joins the merge and chunk passes instead of holding one workgroup
-// for several serial chunk sorts.
-template <bool PACKED>
-__global__ __launch_bounds__(kSortThreads) void k_sort_super(int tiles_x, int tiles_y, int sxn,
-                                                             const int *__restrict__ offsets,
-                                                             unsigned long long *__restrict__ keys,
-                                                             const uint2 *__restrict__ rect,
-                                                             int *__restrict__ tile_counts,
-                                                             int *__restrict__ big_list, int *__restrict__ stats,
-                                                             int *__restrict__ huge_list,
-                                                             int *__restrict__ huge_stats, int huge_th) {
-    __shared__ unsigned long long s[kChunk];
-    __shared__ int s_tc[kSuper * kSuper];
-    const int t = blockIdx.x;
-    const int start = offsets[t], end = offsets[t + 1];
-    const int cnt = end - start;
-    const int stx = (t % sxn) * kSuper, sty = (t / sxn) * kSuper;
-    if (threadIdx.x < kSuper * kSuper) s_tc[threadIdx.x] = 0;
-    __syncthreads();
-    if (cnt <= huge_th) count_tiles<PACKED>(keys + start, cnt, stx, sty, rect, s_tc);
-    if (threadIdx.x < kSuper * kSuper) {
-        const int tx = stx + (int)threadIdx.x % kSuper, ty = sty + (int)threadIdx.x / kSuper;
-        if (tx < tiles_x && ty < tiles_y) tile_counts[ty * tiles_x + tx] = s_tc[threadIdx.x];
+// A thread's counts of the super-tile's 16 tiles, one byte per column of
+// each row: at most 255 keys per thread.
+struct TileCounts {
+    uint32_t row[kSuper] = {0u, 0u, 0u, 0u};
+    __device__ __forceinline__ void add(const int4 &r) {
+        // bytes x0 .. x1 - 1 (0 <= x0 < x1 <= 4)
+        const uint32_t cols = (0x01010101u << (8 * r.x)) & (0x01010101u >> (8 * (kSuper - r.y)));
+#pragma unroll
+        for (int y = 0; y < kSuper; ++y) row[y] += (y >= r.z && y < r.w) ? cols : 0u;
     }
-    if (cnt > kChunk && threadIdx.x == 0) big_list[atomicAdd(&stats[2], 1)] = t;
-    if (cnt > huge_th) {
+    // Adds the wave's sums to s_tc[16] (two 16-bit sums per shuffle: at most
+    // 64 x 255).
+    __device__ __forceinline__ void flush(int *s_tc) const {
+#pragma unroll
+        for (int y = 0; y < kSuper; ++y) {
+#pragma unroll
+            for (int o = 0; o < 2; ++o) {
+                uint32_t v = (row[y] >> (8 * o)) & 0x00ff00ffu;
+#pragma unroll
+                for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+                if ((threadIdx.x & 63) == 0 && v) {
+                    if (v & 0xffffu) atomicAdd(&s_tc[kSuper * y + o], (int)(v & 0xffffu));
+                    if (v >> 16) atomicAdd(&s_tc[kSuper * y + 2 + o], (int)(v >> 16));
+                }
+            }
+        }
+    }
+};
+
+// Counts the entries of the super-tile's 16 tiles into tile_counts, then
+// sorts the super-tile list in place, for lists of above and up to CAP keys
+// (the others belong to another launch).  With CAP = kRun longer lists are
+// queued on huge_list (their tile counts zeroed): k_sort_runs sorts their
+// runs on many workgroups, and after the merge passes k_count_chunks /
+// k_emit_chunks count and emit them chunk by chunk.
+template <bool PACKED, int CAP, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_sort_super(int tiles_x, int tiles_y, int sxn,
+                                                        const int *__restrict__ offsets,
+                                                        unsigned long long *__restrict__ keys,
+                                                        const uint2 *__restrict__ rect,
+                                                        int *__restrict__ tile_counts, int *__restrict__ huge_list,
+                                                        int *__restrict__ huge_stats, int above) {
+    using Sort = RunSort<CAP, THREADS>;
+    __shared__ typename Sort::Lds L;
+    const int t = blockIdx.x;
+    const int start = offsets[t], cnt = offsets[t + 1] - start;
+    if (cnt <= above || (CAP < kRun && cnt > CAP)) return;
+    const int stx = (t % sxn) * kSuper, sty = (t / sxn) * kSuper;
+    Sort st;
+    if (threadIdx.x < kTiles) L.tc[threadIdx.x] = 0;
+    if (cnt <= CAP) st.load(keys + start, cnt);
+    __syncthreads();
+    if (cnt > 0 && cnt <= CAP) {
+        TileCounts tc;
+#pragma unroll
+        for (int j = 0; j < Sort::K; ++j)
+            if (j * THREADS + (int)threadIdx.x < cnt) tc.add(key_rect<PACKED>(st.k[j], stx, sty, rect));
+        tc.flush(L.tc);
+    }
+    __syncthreads();
+    if (threadIdx.x < kTiles) {
+        const int tx = stx + (int)threadIdx.x % kSuper, ty = sty + (int)threadIdx.x / kSuper;
+        if (tx < tiles_x && ty < tiles_y) tile_counts[ty * tiles_x + tx] = L.tc[threadIdx.x];
+    }
+    if (cnt > CAP) {
         if (threadIdx.x == 0) huge_list[atomicAdd(&huge_stats[0], 1)] = t;
         return;
     }
-    if (cnt <= 1) return;
-    for (int c0 = start; c0 < end; c0 += kChunk) {
-        const int c = min(kChunk, end - c0);
-        lds_bitonic(s, keys + c0, c);
-        for (int i = threadIdx.x; i < c; i += kSortThreads) keys[c0 + i] = s[sort_slot(i)];
-        __syncthreads();
-    }
+    if (cnt > 1) st.sort(L, keys + start, cnt);
 }
 
 // Unit numbering of lists of super-tiles: base[b] = the number of
@@ -568,25 +724,26 @@ __device__ __forceinline__ int list_of_unit(const int *__restrict__ base, int n,
     return lo;
 }
 
-// Sorts every kChunk run of the huge lists in LDS, one run per workgroup
-// iteration: the grid strides over the runs of all the lists (chunk_base
-// numbers them), so every run has its own workgroup whatever the lists'
-// lengths.
-__global__ __launch_bounds__(kSortThreads) void k_sort_chunks(const int *__restrict__ offsets,
-                                                              const int *__restrict__ big_list,
-                                                              const int *__restrict__ stats,
-                                                              const int *__restrict__ chunk_base,
-                                                              unsigned long long *__restrict__ keys) {
-    __shared__ unsigned long long s[kChunk];
+// Sorts every kRun run of the huge lists, one run per workgroup iteration:
+// the grid strides over the kChunk chunks of all the lists (chunk_base
+// numbers them) and a run belongs to its first chunk.
+__global__ __launch_bounds__(1024) void k_sort_runs(const int *__restrict__ offsets,
+                                                    const int *__restrict__ huge_list,
+                                                    const int *__restrict__ stats,
+                                                    const int *__restrict__ chunk_base,
+                                                    unsigned long long *__restrict__ keys) {
+    using Sort = RunSort<kRun, 1024>;
+    __shared__ Sort::Lds L;
     const int nbig = stats[0], nchunks = stats[1];
     for (int g = blockIdx.x; g < nchunks; g += gridDim.x) {
         const int b = list_of_unit(chunk_base, nbig, g);
-        const int t = big_list[b];
-        const int start = offsets[t], cnt = offsets[t + 1] - start;
-        const int c0 = (g - chunk_base[b]) * kChunk;
-        const int c = min(kChunk, cnt - c0);
-        lds_bitonic(s, keys + start + c0, c);
-        for (int i = threadIdx.x; i < c; i += kSortThreads) keys[start + c0 + i] = s[sort_slot(i)];
+        const int ch = g - chunk_base[b];
+        if (ch % (kRun / kChunk)) continue;
+        const int t = huge_list[b];
+        const int c0 = offsets[t] + ch * kChunk, c = min(kRun, offsets[t + 1] - c0);
+        Sort st;
+        st.load(keys + c0, c);
+        if (c > 1) st.sort(L, keys + c0, c);
         __syncthreads();
     }
 }
@@ -594,31 +751,33 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_chunks(const int *__restr
 // Tile counts of every kChunk chunk of the merged huge lists:
 // chunk_counts[chunk_base[b] + c][16], summed into tile_counts.
 template <bool PACKED>
-__global__ __launch_bounds__(kSortThreads) void k_count_chunks(int tiles_x, int tiles_y, int sxn,
-                                                               const int *__restrict__ offsets,
-                                                               const int *__restrict__ big_list,
-                                                               const int *__restrict__ stats,
-                                                               const int *__restrict__ chunk_base,
-                                                               const unsigned long long *__restrict__ skeys,
-                                                               const unsigned long long *__restrict__ keys2,
-                                                               const uint2 *__restrict__ rect,
-                                                               int *__restrict__ chunk_counts,
-                                                               int *__restrict__ tile_counts) {
-    __shared__ int s_tc[kSuper * kSuper];
+__global__ __launch_bounds__(256) void k_count_chunks(int tiles_x, int tiles_y, int sxn,
+                                                      const int *__restrict__ offsets,
+                                                      const int *__restrict__ huge_list,
+                                                      const int *__restrict__ stats,
+                                                      const int *__restrict__ chunk_base,
+                                                      const unsigned long long *__restrict__ skeys,
+                                                      const unsigned long long *__restrict__ keys2,
+                                                      const uint2 *__restrict__ rect,
+                                                      int *__restrict__ chunk_counts, int *__restrict__ tile_counts) {
+    __shared__ int s_tc[kTiles];
     const int nbig = stats[0], nchunks = stats[1];
     for (int g = blockIdx.x; g < nchunks; g += gridDim.x) {
         const int b = list_of_unit(chunk_base, nbig, g);
-        const int t = big_list[b];
+        const int t = huge_list[b];
         const int start = offsets[t], cnt = offsets[t + 1] - start;
         const int stx = (t % sxn) * kSuper, sty = (t / sxn) * kSuper;
-        const int c = g - chunk_base[b];
-        const unsigned long long *__restrict__ keys = merged_keys(cnt, skeys, keys2);
-        if (threadIdx.x < kSuper * kSuper) s_tc[threadIdx.x] = 0;
+        const int c = g - chunk_base[b], n = min(kChunk, cnt - c * kChunk);
+        const unsigned long long *__restrict__ keys = merged_keys(cnt, skeys, keys2) + start + c * kChunk;
+        if (threadIdx.x < kTiles) s_tc[threadIdx.x] = 0;
         __syncthreads();
-        count_tiles<PACKED>(keys + start + c * kChunk, min(kChunk, cnt - c * kChunk), stx, sty, rect, s_tc);
-        if (threadIdx.x < kSuper * kSuper) {
+        TileCounts tc;  // kChunk / 256 = 16 keys per thread
+        for (int e = threadIdx.x; e < n; e += 256) tc.add(key_rect<PACKED>(keys[e], stx, sty, rect));
+        tc.flush(s_tc);
+        __syncthreads();
+        if (threadIdx.x < kTiles) {
             const int v = s_tc[threadIdx.x];
-            chunk_counts[(size_t)g * (kSuper * kSuper) + threadIdx.x] = v;
+            chunk_counts[(size_t)g * kTiles + threadIdx.x] = v;
             const int tx = stx + (int)threadIdx.x % kSuper, ty = sty + (int)threadIdx.x / kSuper;
             if (v && tx < tiles_x && ty < tiles_y) atomicAdd(&tile_counts[ty * tiles_x + tx], v);
         }
@@ -626,9 +785,9 @@ __global__ __launch_bounds__(kSortThreads) void k_count_chunks(int tiles_x, int 
     }
 }
 
-// ---- merge passes over the lists longer than kChunk ------------------------
+// ---- merge passes over the lists longer than kRun ------------------------
 //
-// Runs of L sorted keys are merged pairwise, L = kChunk, 2 kChunk, ... .  A
+// Runs of L sorted keys are merged pairwise, L = kRun, 2 kRun, ... .  A
 // pass is a merge path (Odeh et al., "Merge Path -- parallel merging made
 // simple", 2012): the merged output of a pair is cut into tiles of kMergeTile
 // keys; a workgroup finds where its tile's first and last diagonal cross the
@@ -687,16 +846,17 @@ __device__ __forceinline__ int merge_split_wave(const K *__restrict__ A, int la,
 }
 
 __global__ __launch_bounds__(256) void k_merge_path(int L, const int *__restrict__ offsets,
-                                                    const int *__restrict__ big_list, const int *__restrict__ stats,
+                                                    const int *__restrict__ huge_list,
+                                                    const int *__restrict__ nlists, const int *__restrict__ ntiles_p,
                                                     const int *__restrict__ merge_base,
                                                     const unsigned long long *__restrict__ src,
                                                     unsigned long long *__restrict__ dst) {
     __shared__ unsigned long long s_k[kMergeTile];
     __shared__ int s_split[2];
-    const int nbig = stats[2], ntiles = stats[3];
+    const int nbig = *nlists, ntiles = *ntiles_p;
     for (int g = blockIdx.x; g < ntiles; g += gridDim.x) {
         const int b = list_of_unit(merge_base, nbig, g);
-        const int t = big_list[b];
+        const int t = huge_list[b];
         const int start = offsets[t], cnt = offsets[t + 1] - start;
         if (cnt <= L) continue;  // merged by an earlier pass
         // 2L is a multiple of kMergeTile, so no tile straddles two pairs
@@ -740,129 +900,123 @@ __global__ __launch_bounds__(256) void k_merge_path(int L, const int *__restrict
     }
 }
 
-constexpr int kWin = 2048;  // super-list entries staged in LDS per window
+// ---- emission ---------------------------------------------------------------
+//
+// One workgroup of 16 waves per sorted super-tile list (or 4096-key chunk of
+// a huge one), one wave per tile: a window of the list is staged in LDS as
+// (splat, mask of the tiles it covers), and every wave walks the masks 64
+// entries at a time, four steps in flight, writing the splats of its tile in
+// list order (a lane's slot is the popcount of the covering lanes below it).
+// Bound by the latency of that walk: with a wave per tile row, four tiles
+// each, the 294 lists of a 1297 x 840 frame of 500k splats took 43 us; 18 us
+// now (5187 x 3361, 3M splats: 93 -> 78 us).
+constexpr int kWin = kChunk, kEmitThreads = 64 * kTiles;
+struct EmitLds {
+    int gid[kWin];
+    unsigned short mask[kWin];
+};
 
 // Filters the sorted super-list entries skeys[0, cnt) of the super-tile at
-// tile (stx, sty) into the id lists of its tiles: wave w emits the 4 tiles of
-// row w; out[lx] is the tile's list position of the first entry (-1 for a
-// tile outside the image).  Within a 64-entry chunk a lane's output slot is
-// the popcount of the covering lanes below it, so each tile list keeps the
-// super-list (depth, id) order.  Block-uniform.
+// tile (stx, sty) into the id lists of its tiles; out is the position of the
+// first entry in this wave's tile list (-1 for a tile outside the image).
+// Block-uniform.
 template <bool PACKED>
 __device__ __forceinline__ void emit_range(const unsigned long long *__restrict__ skeys, int cnt, int stx, int sty,
-                                           const uint2 *__restrict__ rect, int out[kSuper], int *s_gid,
-                                           unsigned short *s_rr, int *__restrict__ ids) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+                                           const uint2 *__restrict__ rect, int out, EmitLds &L,
+                                           int *__restrict__ ids) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned long long below = (1ull << lane) - 1ull;
     for (int w0 = 0; w0 < cnt; w0 += kWin) {
         const int wn = min(kWin, cnt - w0);
         __syncthreads();
-        for (int k = threadIdx.x; k < wn; k += 256) {
-            const uint32_t lo = (uint32_t)(skeys[w0 + k] & 0xffffffffull);
-            int gid, rx0, rx1, ry0, ry1;
-            if constexpr (PACKED) {
-                gid = (int)(lo >> 8);
-                const int4 lr = unpack_rect(lo & 0xffu);
-                rx0 = lr.x, rx1 = lr.y, ry0 = lr.z, ry1 = lr.w;
-            } else {
-                gid = (int)lo;
-                const uint2 r = rect[gid];
-                const int x0 = r.x & 0xffff, y0 = r.x >> 16, x1 = r.y & 0xffff, y1 = r.y >> 16;
-                rx0 = max(x0 - stx, 0), rx1 = min(x1 - stx, kSuper);
-                ry0 = max(y0 - sty, 0), ry1 = min(y1 - sty, kSuper);
+#pragma unroll
+        for (int q = 0; q < kWin / kEmitThreads; ++q) {
+            const int k = q * kEmitThreads + (int)threadIdx.x;
+            if (k < wn) {
+                const unsigned long long key = skeys[w0 + k];
+                const uint32_t lo = (uint32_t)(key & 0xffffffffull);
+                const int4 r = key_rect<PACKED>(key, stx, sty, rect);
+                // bits x0 .. x1 - 1 of each row, in rows y0 .. y1 - 1
+                const unsigned cols = (0xfu << r.x) & (0xfu >> (kSuper - r.y));
+                const unsigned rows = (0xffffu << (kSuper * r.z)) & (0xffffu >> (kSuper * (kSuper - r.w)));
+                L.gid[k] = (int)(PACKED ? lo >> 8 : lo);
+                L.mask[k] = (unsigned short)((cols * 0x1111u) & rows);
             }
-            s_gid[k] = gid;
-            s_rr[k] = (unsigned short)(rx0 | (rx1 << 4) | (ry0 << 8) | (ry1 << 12));
         }
         __syncthreads();
-        for (int j = 0; j < wn; j += 64) {
-            const int idx = j + lane;
-            const int rr = idx < wn ? s_rr[idx] : 0;
-            const int lw = wave;
-            const bool row_in = ((rr >> 8) & 15) <= lw && lw < ((rr >> 12) & 15);
-            const int rx0 = rr & 15, rx1 = (rr >> 4) & 15;
-            const int gid = idx < wn ? s_gid[idx] : 0;
+        if (out < 0) continue;  // uniform over the wave
+        for (int j = 0; j < wn; j += 256) {
+            bool cov[4];
+            int gid[4];
 #pragma unroll
-            for (int lx = 0; lx < kSuper; ++lx) {
-                const bool cov = row_in && rx0 <= lx && lx < rx1;
-                const unsigned long long bal = __ballot(cov);
-                if (cov && out[lx] >= 0) ids[out[lx] + __popcll(bal & below)] = gid;
-                if (out[lx] >= 0) out[lx] += __popcll(bal);
+            for (int u = 0; u < 4; ++u) {
+                const int k = j + 64 * u + lane;
+                cov[u] = k < wn && ((L.mask[min(k, kWin - 1)] >> wave) & 1u);
+                gid[u] = L.gid[min(k, kWin - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned long long bal = __ballot(cov[u]);
+                if (cov[u]) ids[out + __popcll(bal & below)] = gid[u];
+                out += __popcll(bal);
             }
         }
     }
 }
 
-// Emits each super-tile list of at most huge_th entries into its 16 tile
-// lists (longer lists: k_emit_chunks).
+// Emits each super-tile list of at most kRun entries into its 16 tile lists
+// (longer lists: k_emit_chunks).
 template <bool PACKED>
-__global__ __launch_bounds__(256) void k_emit_tiles(int tiles_x, int tiles_y, int sxn,
-                                                    const int *__restrict__ soffsets,
-                                                    const unsigned long long *__restrict__ skeys,
-                                                    const unsigned long long *__restrict__ keys2,
-                                                    const uint2 *__restrict__ rect,
-                                                    const int *__restrict__ toffsets, int *__restrict__ ids,
-                                                    int huge_th) {
-    __shared__ int s_gid[kWin];
-    __shared__ unsigned short s_rr[kWin];
+__global__ __launch_bounds__(kEmitThreads) void k_emit_tiles(int tiles_x, int tiles_y, int sxn,
+                                                             const int *__restrict__ soffsets,
+                                                             const unsigned long long *__restrict__ skeys,
+                                                             const uint2 *__restrict__ rect,
+                                                             const int *__restrict__ toffsets,
+                                                             int *__restrict__ ids) {
+    __shared__ EmitLds L;
     const int st = blockIdx.x;
     const int stx = (st % sxn) * kSuper, sty = (st / sxn) * kSuper;
     const int start = soffsets[st], cnt = soffsets[st + 1] - start;
-    if (cnt > huge_th) return;
-    // lists above kChunk went through their merge passes (merged_keys); the
-    // shorter ones were sorted in place
-    const unsigned long long *__restrict__ keys = cnt > kChunk ? merged_keys(cnt, skeys, keys2) : skeys;
-    const int ty = sty + (int)(threadIdx.x >> 6);
-    int out[kSuper];
-#pragma unroll
-    for (int lx = 0; lx < kSuper; ++lx) {
-        const int tx = stx + lx;
-        out[lx] = (tx < tiles_x && ty < tiles_y) ? toffsets[ty * tiles_x + tx] : -1;
-    }
-    emit_range<PACKED>(keys + start, cnt, stx, sty, rect, out, s_gid, s_rr, ids);
+    if (cnt > kRun) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tx = stx + wave % kSuper, ty = sty + wave / kSuper;
+    const int out = (tx < tiles_x && ty < tiles_y) ? toffsets[ty * tiles_x + tx] : -1;
+    emit_range<PACKED>(skeys + start, cnt, stx, sty, rect, out, L, ids);
 }
 
 // Emits every kChunk chunk of the huge lists: a chunk's entries start in
 // each tile list after those of the chunks before it (chunk_counts).
 template <bool PACKED>
-__global__ __launch_bounds__(256) void k_emit_chunks(int tiles_x, int tiles_y, int sxn,
-                                                     const int *__restrict__ soffsets,
-                                                     const int *__restrict__ big_list,
-                                                     const int *__restrict__ stats,
-                                                     const int *__restrict__ chunk_base,
-                                                     const int *__restrict__ chunk_counts,
-                                                     const unsigned long long *__restrict__ skeys,
-                                                     const unsigned long long *__restrict__ keys2,
-                                                     const uint2 *__restrict__ rect,
-                                                     const int *__restrict__ toffsets, int *__restrict__ ids) {
-    __shared__ int s_gid[kWin];
-    __shared__ unsigned short s_rr[kWin];
+__global__ __launch_bounds__(kEmitThreads) void k_emit_chunks(int tiles_x, int tiles_y, int sxn,
+                                                              const int *__restrict__ soffsets,
+                                                              const int *__restrict__ huge_list,
+                                                              const int *__restrict__ stats,
+                                                              const int *__restrict__ chunk_base,
+                                                              const int *__restrict__ chunk_counts,
+                                                              const unsigned long long *__restrict__ skeys,
+                                                              const unsigned long long *__restrict__ keys2,
+                                                              const uint2 *__restrict__ rect,
+                                                              const int *__restrict__ toffsets,
+                                                              int *__restrict__ ids) {
+    __shared__ EmitLds L;
     const int nbig = stats[0], nchunks = stats[1];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     for (int g = blockIdx.x; g < nchunks; g += gridDim.x) {
         const int b = list_of_unit(chunk_base, nbig, g);
-        const int st = big_list[b];
+        const int st = huge_list[b];
         const int stx = (st % sxn) * kSuper, sty = (st / sxn) * kSuper;
         const int start = soffsets[st], cnt = soffsets[st + 1] - start;
-        const int ty = sty + wave;
         const int c = g - chunk_base[b];
-        // entries of this wave's four tiles in the chunks before c
-        int before[kSuper] = {0, 0, 0, 0};
-        for (int k = lane; k < c; k += 64)
+        // entries of this wave's tile in the chunks before c
+        int v = 0;
+        for (int k = lane; k < c; k += 64) v += chunk_counts[(size_t)(chunk_base[b] + k) * kTiles + wave];
 #pragma unroll
-            for (int lx = 0; lx < kSuper; ++lx)
-                before[lx] += chunk_counts[(size_t)(chunk_base[b] + k) * (kSuper * kSuper) + wave * kSuper + lx];
-        int out[kSuper];
-#pragma unroll
-        for (int lx = 0; lx < kSuper; ++lx) {
-            int v = before[lx];
-#pragma unroll
-            for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-            const int tx = stx + lx;
-            out[lx] = (tx < tiles_x && ty < tiles_y) ? toffsets[ty * tiles_x + tx] + v : -1;
-        }
+        for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+        const int tx = stx + wave % kSuper, ty = sty + wave / kSuper;
+        const int out =
+            __builtin_amdgcn_readfirstlane((tx < tiles_x && ty < tiles_y) ? toffsets[ty * tiles_x + tx] + v : -1);
         emit_range<PACKED>(merged_keys(cnt, skeys, keys2) + start + c * kChunk, min(kChunk, cnt - c * kChunk), stx,
-                           sty, rect, out, s_gid, s_rr, ids);
+                           sty, rect, out, L, ids);
     }
 }
 
@@ -907,9 +1061,9 @@ void launch_super_count(hipStream_t s, int n, int tiles_x, int tiles_y, const in
 
 void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int *radii, const uint32_t *rect,
                       const float *depths, const int *super_offsets, const int *super_cm, int super_max,
-                      uint64_t *super_keys, uint64_t *super_keys_tmp, int *big_list, int *super_stats,
-                      int *huge_list, int *huge_stats, int *chunk_base, int *chunk_counts, int *merge_base,
-                      int total_keys, int *tile_counts, int *tile_offsets, int *tile_stats, int *tile_temp, int *ids,
+                      uint64_t *super_keys, uint64_t *super_keys_tmp, int *super_stats, int *huge_list,
+                      int *huge_stats, int *chunk_base, int *chunk_counts, int *merge_base, int total_keys,
+                      int *tile_counts, int *tile_offsets, int *tile_stats, int *tile_temp, int *ids,
                       bool force_wide_keys, const DeepScan *deep) {
     const int sxn = (tiles_x + kSuper - 1) / kSuper, syn = (tiles_y + kSuper - 1) / kSuper, NS = sxn * syn;
     const int T = tiles_x * tiles_y;
@@ -922,48 +1076,66 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
     if (n > 0)
         hipLaunchKernelGGL(packed ? k_scatter_super<true> : k_scatter_super<false>, dim3(blocks), dim3(kBinThreads), 0,
                            s, n, chunk, sxn, NS, radii, r2, depths, super_offsets, super_cm, k);
-    const bool big = bin_chunk_parallel(super_max, NS);
-    const int huge_th = big ? kChunk : kHuge;
-    hipLaunchKernelGGL(packed ? k_sort_super<true> : k_sort_super<false>, dim3(NS), dim3(kSortThreads), 0, s, tiles_x,
-                       tiles_y, sxn, super_offsets, k, r2, tile_counts, big_list, super_stats, huge_list, huge_stats,
-                       huge_th);
-    // huge lists: kChunk runs sorted on many workgroups, then merged.  The
+    // Workgroups of the three sorts per CU: four of 4096 keys (40 KB of LDS,
+    // 512 threads), two of 8192 (80 KB, 1024 threads), one of kRun (145 KB).
+    // One launch of the smallest that takes the frame's longest list, as long
+    // as all its workgroups run at once; otherwise the many lists of at most
+    // 4096 keys go first, on the small sort, and the larger one takes the
+    // rest (its other workgroups end at once): 4346 lists 87 + 22 us against
+    // 200 us all on the middle sort.
+    const auto sort = [&](auto kernel, int threads, int above) {
+        hipLaunchKernelGGL(kernel, dim3(NS), dim3(threads), 0, s, tiles_x, tiles_y, sxn, super_offsets, k, r2,
+                           tile_counts, huge_list, huge_stats, above);
+    };
+    constexpr int kCus = 256;
+    const bool mid = super_max <= 8192;
+    int above = -1;
+    if (super_max <= 4096 || NS > (mid ? 2 * kCus : kCus)) {
+        sort(packed ? k_sort_super<true, 4096, 512> : k_sort_super<false, 4096, 512>, 512, above);
+        above = 4096;
+    }
+    if (super_max > 4096) {
+        if (mid)
+            sort(packed ? k_sort_super<true, 8192, 1024> : k_sort_super<false, 8192, 1024>, 1024, above);
+        else
+            sort(packed ? k_sort_super<true, kRun, 1024> : k_sort_super<false, kRun, 1024>, 1024, above);
+    }
+    // huge lists: kRun runs sorted on many workgroups, then merged.  The
     // chunk and merge-tile kernels stride over units numbered across all
     // their lists; their grids cover at most total_keys / unit + NS units
     // (each list rounds up once)
-    const int big_grid = (int)std::min<int64_t>(4096, (int64_t)total_keys / kChunk + NS);
-    if (super_max > kChunk) {
+    const bool huge = super_max > kRun;
+    const int huge_grid = (int)std::min<int64_t>(4096, (int64_t)total_keys / kChunk + NS);
+    if (huge) {
         const UnitList chunks{huge_list, huge_stats, kChunk, chunk_base, huge_stats + 1};
-        const UnitList tiles{big_list, super_stats + 2, kMergeTile, merge_base, super_stats + 3};
-        hipLaunchKernelGGL(k_list_prep, dim3(1), dim3(1024), 0, s, super_offsets, big ? chunks : UnitList{}, tiles);
-    }
-    if (big)
-        hipLaunchKernelGGL(k_sort_chunks, dim3(big_grid), dim3(kSortThreads), 0, s, super_offsets, huge_list,
-                           huge_stats, chunk_base, k);
-    unsigned long long *src = k, *dst = kt;
-    const int merge_grid = (int)std::min<int64_t>(8192, (int64_t)total_keys / kMergeTile + NS);
-    for (int L = kChunk; L < super_max; L <<= 1) {
-        hipLaunchKernelGGL(k_merge_path, dim3(merge_grid), dim3(256), 0, s, L, super_offsets, big_list, super_stats,
-                           merge_base, src, dst);
-        std::swap(src, dst);
-    }
-    // each list longer than kChunk ends in the buffer its last pass wrote
-    // (merged_keys); the emission reads it there
-    if (big)
-        hipLaunchKernelGGL(packed ? k_count_chunks<true> : k_count_chunks<false>, dim3(big_grid), dim3(kSortThreads), 0, s,
+        const UnitList tiles{huge_list, huge_stats, kMergeTile, merge_base, super_stats + 3};
+        hipLaunchKernelGGL(k_list_prep, dim3(1), dim3(1024), 0, s, super_offsets, chunks, tiles);
+        hipLaunchKernelGGL(k_sort_runs, dim3(huge_grid), dim3(1024), 0, s, super_offsets, huge_list, huge_stats,
+                           chunk_base, k);
+        unsigned long long *src = k, *dst = kt;
+        const int merge_grid = (int)std::min<int64_t>(8192, (int64_t)total_keys / kMergeTile + NS);
+        for (int L = kRun; L < super_max; L <<= 1) {
+            hipLaunchKernelGGL(k_merge_path, dim3(merge_grid), dim3(256), 0, s, L, super_offsets, huge_list,
+                               huge_stats, super_stats + 3, merge_base, src, dst);
+            std::swap(src, dst);
+        }
+        // each list ends in the buffer its last pass wrote (merged_keys); the
+        // emission reads it there
+        hipLaunchKernelGGL(packed ? k_count_chunks<true> : k_count_chunks<false>, dim3(huge_grid), dim3(256), 0, s,
                            tiles_x, tiles_y, sxn, super_offsets, huge_list, huge_stats, chunk_base, k, kt, r2,
                            chunk_counts, tile_counts);
+    }
     launch_scan_counts(s, T, tile_counts, tile_offsets, nullptr, tile_stats, tile_temp);
     if (deep) {
         launch_deep_tiles(s, T, tile_offsets, deep->len, deep->list, deep->count);
         (void)hipMemcpyAsync(deep->host_count, deep->count, sizeof(int), hipMemcpyDeviceToHost, s);
     }
-    hipLaunchKernelGGL(packed ? k_emit_tiles<true> : k_emit_tiles<false>, dim3(NS), dim3(256), 0, s, tiles_x, tiles_y,
-                       sxn, super_offsets, k, kt, r2, tile_offsets, ids, huge_th);
-    if (big)
-        hipLaunchKernelGGL(packed ? k_emit_chunks<true> : k_emit_chunks<false>, dim3(big_grid), dim3(256), 0, s, tiles_x,
-                           tiles_y, sxn, super_offsets, huge_list, huge_stats, chunk_base, chunk_counts, k, kt, r2,
-                           tile_offsets, ids);
+    hipLaunchKernelGGL(packed ? k_emit_tiles<true> : k_emit_tiles<false>, dim3(NS), dim3(kEmitThreads), 0, s, tiles_x,
+                       tiles_y, sxn, super_offsets, k, r2, tile_offsets, ids);
+    if (huge)
+        hipLaunchKernelGGL(packed ? k_emit_chunks<true> : k_emit_chunks<false>, dim3(huge_grid), dim3(kEmitThreads), 0,
+                           s, tiles_x, tiles_y, sxn, super_offsets, huge_list, huge_stats, chunk_base, chunk_counts, k,
+                           kt, r2, tile_offsets, ids);
 }
 
 }  // namespace mskern

@@ -54,7 +54,8 @@ void launch_tiles_hit(hipStream_t s, const uint32_t *rect, const int *radii, int
 // NS = sxn * syn.  Scan temporaries: tile_scan_temp_ints(count) ints.
 int64_t tile_scan_temp_ints(int T);
 // (splat, super-tile) pair counts -> super_counts[NS], super_offsets[NS + 1];
-// super_stats = {pairs, largest list, long-list count}, zero on entry.
+// super_stats = {pairs, largest list, -, merge tiles of the huge lists},
+// zero on entry.
 // super_cm (kBinMaxBlocks x NS ints) receives the per-(workgroup,
 // super-tile) key offsets that launch_bin_tiles places the keys at.
 void launch_super_count(hipStream_t s, int n, int tiles_x, int tiles_y, const int *radii, const uint32_t *rect,
@@ -62,12 +63,11 @@ void launch_super_count(hipStream_t s, int n, int tiles_x, int tiles_y, const in
 constexpr int kBinMaxBlocks = 256;
 // Scatter, per-super-tile sort, tile counts and offsets (tile_offsets[T + 1],
 // tile_stats = {intersections, largest tile}, zero on entry) and the
-// per-tile sorted gaussian ids.  When super_max > 4096 the long lists need
-// super_keys_tmp (the size of super_keys) and merge_base[NS], and
-// super_stats[3] receives their merge-tile count; when
-// bin_chunk_parallel(super_max, NS) huge_list[NS], huge_stats[2] (zero on
-// entry), chunk_base[NS] and chunk_counts[big_chunk_ints(total, NS)].
-// total_keys = the pair count (super_stats[0]).
+// per-tile sorted gaussian ids.  When bin_huge_lists(super_max) the long
+// lists need super_keys_tmp (the size of super_keys), huge_list[NS],
+// huge_stats[2] (zero on entry), chunk_base[NS], merge_base[NS] and
+// chunk_counts[huge_chunk_ints(total, NS)], and super_stats[3] receives
+// their merge-tile count.  total_keys = the pair count (super_stats[0]).
 // The deep-tile scan launch_bin_tiles queues once the tile offsets exist
 // (before the emission kernels): the tiles with at least `len` entries into
 // `list`, their number into *count, copied to *host_count.
@@ -77,23 +77,20 @@ struct DeepScan {
 };
 void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int *radii, const uint32_t *rect,
                       const float *depths, const int *super_offsets, const int *super_cm, int super_max,
-                      uint64_t *super_keys, uint64_t *super_keys_tmp, int *big_list, int *super_stats,
-                      int *huge_list, int *huge_stats, int *chunk_base, int *chunk_counts, int *merge_base,
-                      int total_keys, int *tile_counts, int *tile_offsets, int *tile_stats, int *tile_temp, int *ids,
+                      uint64_t *super_keys, uint64_t *super_keys_tmp, int *super_stats, int *huge_list,
+                      int *huge_stats, int *chunk_base, int *chunk_counts, int *merge_base, int total_keys,
+                      int *tile_counts, int *tile_offsets, int *tile_stats, int *tile_temp, int *ids,
                       bool force_wide_keys, const DeepScan *deep = nullptr);
-constexpr int kSuperHugeList = 4 * 4096;
-// Whether the super-tile lists above 4096 keys are sorted, counted and
-// emitted chunk-parallel (k_sort_chunks, k_count_chunks, k_emit_chunks):
-// when some list exceeds kSuperHugeList, which a workgroup would otherwise
-// hold for several serial chunk sorts.  (Also taking that path for frames
-// with few super-tiles, e.g. 294 at 1297x840, measured 1-3% slower steps:
-// its extra launches cost more than the serial sorts of lists of <= 16k.)
-inline bool bin_chunk_parallel(int super_max, int /*num_super*/) { return super_max > kSuperHugeList; }
-// Ints of chunk_counts: 16 per 4096-key chunk of the long lists, at most
-// total / 4096 + NS chunks.
-inline int64_t big_chunk_ints(int64_t total_keys, int NS) { return (total_keys / 4096 + NS) * 16; }
 constexpr int kSuperTile = 4;
-constexpr int kSuperSortChunk = 4096;
+// Keys of a super-tile list that one workgroup sorts in LDS, and keys per
+// counting and emission unit of a longer (huge) list.
+constexpr int kSuperSortRun = 16384, kSuperChunk = 4096;
+// Whether some list exceeds kSuperSortRun: those lists are sorted in runs,
+// merged, counted and emitted by many workgroups each.
+inline bool bin_huge_lists(int super_max) { return super_max > kSuperSortRun; }
+// Ints of chunk_counts: 16 per chunk of the huge lists, at most
+// total / kSuperChunk + NS chunks.
+inline int64_t huge_chunk_ints(int64_t total_keys, int NS) { return (total_keys / kSuperChunk + NS) * 16; }
 
 // k_raster.hip
 // blog (msr::BlendLog: a pool of 64-entry chunks of 16-byte entries with

@@ -145,6 +145,44 @@ def test_overflow_tiles_merge_path(wide, orc, eng):
     _assert_bitexact(out["final_idx"], fwd["final_idx"], "final_idx")
 
 
+def _depths(pattern, n, rng):
+    """Camera-axis positions of n splats: spread evenly, all equal, most in a
+    thin slab (buckets drawn again), two exact planes inside a spread, a
+    geometric pile-up (crowded after redrawing too)."""
+    z = rng.uniform(-1.0, 1.0, n)
+    if pattern == "plane":
+        z[:] = 0.25
+    elif pattern == "slab":
+        z[: n - n // 16] = 0.3 + 1e-4 * rng.uniform(size=n - n // 16)
+    elif pattern == "planes":
+        z[: n // 3], z[n // 3: n // 2] = -0.5, 0.5
+    elif pattern == "piled":
+        z = 1.0 - 2.0 ** (-20.0 * rng.uniform(size=n))
+    return z.astype(np.float32)
+
+
+@pytest.mark.parametrize("pattern,wide", [("even", False), ("plane", False), ("slab", False), ("planes", False),
+                                          ("piled", False), ("even", True), ("slab", True)])
+@pytest.mark.parametrize("n", [1, 2, 65, 4096, 4097, 8192, 8193, 16384, 16385])
+def test_super_tile_sort_bitexact(n, pattern, wide, orc, eng):
+    """One super-tile (64 x 64 pixels) whose list has n keys, around the
+    capacities of the in-LDS sorts (4096, 8192, 16384 keys) and with depths
+    that spread, crowd and coincide: the per-tile order is the golden
+    model's."""
+    rng = np.random.default_rng(n)
+    scene = S.make_scene(1, n=n, width=64, height=64, seed=n)
+    scene.means[:, :2] = rng.uniform(-0.8, 0.8, (n, 2)).astype(np.float32)
+    scene.means[:, 2] = _depths(pattern, n, rng)
+    print(f"[sort] n={n} pattern={pattern} wide={wide}", flush=True)
+    E.check(E.lib().msplat_hip_set_wide_keys(1 if wide else 0))
+    try:
+        ocam, proj, bins, fwd, ds, gcam, out = _forward_both(scene, 0, orc, eng)
+    finally:
+        E.check(E.lib().msplat_hip_set_wide_keys(0))
+    _assert_bitexact(E.last("tile_offsets"), bins["tile_offsets"], "tile offsets")
+    _assert_bitexact(E.last("gaussian_ids"), bins["ids"], "per-tile sorted ids")
+
+
 @pytest.mark.parametrize("name", ["blob40k_sh3", "adversarial"])
 def test_wide_binning_keys_bitexact(name, orc, eng):
     """The binning's wide key layout (depth bits << 32 | id, the rectangle
