@@ -81,7 +81,7 @@ struct Engine {
     // quadrant-mask records (msd::MaskRec, 12 floats each; mask_recs())
     DevBuf rec, depths, radii, rect, grads16, colors_raw;
     // per-tile
-    DevBuf counts, offsets, stats, scan_tmp;
+    DevBuf counts, offsets, stats, scan_tmp, tile_order;
     DevBuf huge_list, chunk_base, chunk_counts;  // super-tile lists above 16384 keys, their chunk numbering and counts
     DevBuf merge_base;                           // the merge-tile numbering of the huge lists
     DevBuf super_counts, super_offsets, super_cm, super_tmp;  // super_cm: per-(workgroup, super-tile) offsets
@@ -456,13 +456,13 @@ int raster_fwd_locked(bool log, bool full) {
             set_err("the 3DGS mode produces the image and the transmittance only");
             return MSPLAT_E_ARG;
         }
-        mskern::launch_raster3d_fwd(E.stream, E.W, E.H, E.tiles_x, E.tiles_y, P<int>(E.offsets), P<int>(E.ids),
+        mskern::launch_raster3d_fwd(E.stream, E.W, E.H, E.tiles_x, E.tiles_y, P<int>(E.tile_order), P<int>(E.offsets), P<int>(E.ids),
                                     P<float>(E.rec), P<float>(E.rec) + (size_t)E.n * mskern::kRec3Floats, E.bg,
                                     P<float>(E.out_img), P<float>(E.final_Ts), log ? &blog : nullptr);
         E.log_valid = E.log_valid || log;
         return MSPLAT_OK;
     }
-    mskern::launch_raster_fwd(E.stream, E.W, E.H, E.tiles_x, E.tiles_y, P<int>(E.offsets), P<int>(E.ids),
+    mskern::launch_raster_fwd(E.stream, E.W, E.H, E.tiles_x, E.tiles_y, P<int>(E.tile_order), P<int>(E.offsets), P<int>(E.ids),
                               P<float>(E.rec), mask_recs(), E.bg, P<float>(E.out_img), P<float>(E.final_Ts),
                               P<int>(E.final_idx),
                               P<float>(E.out_depth), P<float>(E.out_normal), P<float>(E.out_alpha),
@@ -507,6 +507,7 @@ int forward_locked(const MsplatCamera *cam, const MsplatGaussians *g, const floa
     CHECK(ensure(E.counts, (size_t)T * 4));
     CHECK(ensure(E.scan_tmp, (size_t)mskern::tile_scan_temp_ints(T) * 4));
     CHECK(ensure(E.offsets, (size_t)(T + 1) * 4));
+    CHECK(ensure(E.tile_order, (size_t)mskern::tile_order_ints(cam->tiles_x, cam->tiles_y) * 4));
     const int sxn = (cam->tiles_x + mskern::kSuperTile - 1) / mskern::kSuperTile;
     const int syn = (cam->tiles_y + mskern::kSuperTile - 1) / mskern::kSuperTile;
     const int NS = sxn * syn;
@@ -599,7 +600,7 @@ int forward_locked(const MsplatCamera *cam, const MsplatGaussians *g, const floa
                              P<uint64_t>(E.keys), P<uint64_t>(E.keys_tmp), P<int>(E.stats) + 4, P<int>(E.huge_list),
                              P<int>(E.stats) + 12, P<int>(E.chunk_base), P<int>(E.chunk_counts),
                              P<int>(E.merge_base), S_total, P<int>(E.counts), P<int>(E.offsets), P<int>(E.stats),
-                             P<int>(E.scan_tmp), P<int>(E.ids), E.wide_keys, scan_deep ? &dscan : nullptr);
+                             P<int>(E.scan_tmp), P<int>(E.ids), I, P<int>(E.tile_order), E.wide_keys, scan_deep ? &dscan : nullptr);
     E.n_deep = 0;
     if (scan_deep) {
         HIPC(hipStreamSynchronize(s));
@@ -773,7 +774,7 @@ void msplat_hip_cleanup(void) {
     (void)hipStreamSynchronize(E.stream);
     if (E.deep_stream) (void)hipStreamSynchronize(E.deep_stream);
     DevBuf *all[] = {&E.rec, &E.depths, &E.radii, &E.rect, &E.grads16, &E.colors_raw, &E.counts, &E.scan_tmp, &E.super_counts, &E.super_offsets, &E.super_cm, &E.super_tmp, &E.offsets,
-                     &E.stats, &E.huge_list, &E.chunk_base, &E.chunk_counts, &E.merge_base, &E.keys, &E.keys_tmp, &E.ids, &E.blend_log, &E.t_ckpt, &E.wave_cnt, &E.selfcheck, &E.out_img, &E.final_Ts,
+                     &E.stats, &E.tile_order, &E.huge_list, &E.chunk_base, &E.chunk_counts, &E.merge_base, &E.keys, &E.keys_tmp, &E.ids, &E.blend_log, &E.t_ckpt, &E.wave_cnt, &E.selfcheck, &E.out_img, &E.final_Ts,
                      &E.final_idx, &E.out_depth, &E.out_normal, &E.out_alpha, &E.out_median, &E.out_dist,
                      &E.dL_dimg, &E.gm1, &E.gs1, &E.gs12, &E.partials, &E.loss, &E.dmeans, &E.dscales,
                      &E.dquats, &E.dmean2d, &E.dfdc, &E.dfrest, &E.dens_flags, &E.dens_scan, &E.dens_keep, &E.dens_ws, &E.deep_list, &E.deep_pos, &E.deep_tb, &E.deep_cnt, &E.log_table, &E.log_ctr, &E.pair_counter,
@@ -1122,7 +1123,7 @@ static int train_step_once(const MsplatCamera *cam, const MsplatGaussians *g, co
     // the layout the logging forward planned (a new plan could reallocate
     // the pool under the log)
     const msr::BlendLog blog = E.log_desc;
-    const bool t_moments = mskern::launch_raster_bwd(s, W, H, cam->tiles_x, cam->tiles_y, P<int>(E.offsets), blog,
+    const bool t_moments = mskern::launch_raster_bwd(s, W, H, cam->tiles_x, cam->tiles_y, P<int>(E.tile_order), P<int>(E.offsets), blog,
                               P<float>(E.rec), bg, P<float>(E.final_Ts),
                               P<int>(E.final_idx), P<float>(E.dL_dimg), nullptr, nullptr, nullptr, nullptr, nullptr,
                               ddist_uniform, P<float>(E.grads16), deep);
@@ -1227,7 +1228,7 @@ static int train_step3d_once(const MsplatCamera *cam, const MsplatGaussians *g, 
     // the layout the logging forward planned (a new plan could reallocate
     // the pool under the log)
     const msr::BlendLog blog = E.log_desc;
-    mskern::launch_raster3d_bwd(s, W, H, cam->tiles_x, cam->tiles_y, P<int>(E.offsets), blog, P<float>(E.rec), bg,
+    mskern::launch_raster3d_bwd(s, W, H, cam->tiles_x, cam->tiles_y, P<int>(E.tile_order), P<int>(E.offsets), blog, P<float>(E.rec), bg,
                                 P<float>(E.final_Ts), P<float>(E.dL_dimg), P<float>(E.grads16));
     stage_mark(ST_PROJECT_BWD);
     if (adam) {
@@ -1518,7 +1519,7 @@ int msplat_hip_raster_bwd(const float *dL_dimg, const float *dL_ddepth, const fl
     // the pool under the log)
     const msr::BlendLog blog = E.log_desc;
     const bool t_moments = mskern::launch_raster_bwd(
-        E.stream, E.W, E.H, E.tiles_x, E.tiles_y, P<int>(E.offsets), blog, P<float>(E.rec), E.bg,
+        E.stream, E.W, E.H, E.tiles_x, E.tiles_y, P<int>(E.tile_order), P<int>(E.offsets), blog, P<float>(E.rec), E.bg,
         P<float>(E.final_Ts), P<int>(E.final_idx), dL_dimg, dL_ddepth, dL_dalpha, dL_dnormal, dL_dmedian, dL_ddist,
         0.0f, grads16, deep);
     if (t_moments) mskern::launch_finish_image_grads(E.stream, E.n, P<float>(E.rec), grads16);

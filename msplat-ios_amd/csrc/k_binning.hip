@@ -964,17 +964,61 @@ __device__ __forceinline__ void emit_range(const unsigned long long *__restrict_
     }
 }
 
+// The rasterizers' order of the tiles: workgroup b takes order[b] (-1: none).
+// Slot k of XCD x is workgroup 8 k + x, whose tile xcd_strip_tile deals; an
+// XCD's slots are put in order of their lists' lengths (sixteen classes of a
+// quarter of the frame's mean, longest first), so that the tiles that take
+// several times as long as the rest are not still running after them.  One
+// workgroup per XCD.  With the blob scene of 500k splats at 1297 x 840 the
+// render forward takes 205 us instead of 228, at 200k splats the full-output
+// forward 229 instead of 254; 3M splats at 5187 x 3361 2410 instead of 2466.
+constexpr int kLenClasses = 16;
+__device__ __forceinline__ void order_tiles(int x, int tiles_x, int tiles_y, int quarter,
+                                            const int *__restrict__ toffsets, int *s_n, int *__restrict__ order) {
+    const int slots = msd::xcd_strip_grid(tiles_x, tiles_y) / 8;
+    const auto bucket = [&](int k, int &tile) {
+        tile = msd::xcd_strip_tile(8 * k + x, tiles_x, tiles_y);
+        if (tile < 0) return kLenClasses;  // padding comes last
+        return kLenClasses - 1 - min(kLenClasses - 1, (toffsets[tile + 1] - toffsets[tile]) / quarter);
+    };
+    if (threadIdx.x <= kLenClasses) s_n[threadIdx.x] = 0;
+    __syncthreads();
+    for (int k = threadIdx.x; k < slots; k += kEmitThreads) {
+        int tile;
+        atomicAdd(&s_n[bucket(k, tile)], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int c = 0, run = 0; c <= kLenClasses; ++c) {
+            const int v = s_n[c];
+            s_n[c] = run;
+            run += v;
+        }
+    __syncthreads();
+    for (int k = threadIdx.x; k < slots; k += kEmitThreads) {
+        int tile;
+        const int b = bucket(k, tile);
+        order[8 * atomicAdd(&s_n[b], 1) + x] = tile;
+    }
+}
+
 // Emits each super-tile list of at most kRun entries into its 16 tile lists
-// (longer lists: k_emit_chunks).
+// (longer lists: k_emit_chunks).  The first eight workgroups order the tiles
+// for the rasterizers (order_tiles) meanwhile.
 template <bool PACKED>
 __global__ __launch_bounds__(kEmitThreads) void k_emit_tiles(int tiles_x, int tiles_y, int sxn,
                                                              const int *__restrict__ soffsets,
                                                              const unsigned long long *__restrict__ skeys,
                                                              const uint2 *__restrict__ rect,
                                                              const int *__restrict__ toffsets,
-                                                             int *__restrict__ ids) {
+                                                             int *__restrict__ ids, int tiles_quarter,
+                                                             int *__restrict__ order) {
     __shared__ EmitLds L;
-    const int st = blockIdx.x;
+    if (blockIdx.x < 8) {
+        order_tiles(blockIdx.x, tiles_x, tiles_y, tiles_quarter, toffsets, L.gid, order);
+        return;
+    }
+    const int st = blockIdx.x - 8;
     const int stx = (st % sxn) * kSuper, sty = (st / sxn) * kSuper;
     const int start = soffsets[st], cnt = soffsets[st + 1] - start;
     if (cnt > kRun) return;
@@ -1024,6 +1068,8 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_chunks(int tiles_x, int t
 
 namespace mskern {
 
+int tile_order_ints(int tiles_x, int tiles_y) { return msd::xcd_strip_grid(tiles_x, tiles_y); }
+
 int64_t tile_scan_temp_ints(int T) { return (T + kScanChunk - 1) / kScanChunk + 1; }
 
 // Exclusive scan of counts[T] into offsets[T + 1] (and cursor[T] if given);
@@ -1064,7 +1110,7 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
                       uint64_t *super_keys, uint64_t *super_keys_tmp, int *super_stats, int *huge_list,
                       int *huge_stats, int *chunk_base, int *chunk_counts, int *merge_base, int total_keys,
                       int *tile_counts, int *tile_offsets, int *tile_stats, int *tile_temp, int *ids,
-                      bool force_wide_keys, const DeepScan *deep) {
+                      int num_isect, int *tile_order, bool force_wide_keys, const DeepScan *deep) {
     const int sxn = (tiles_x + kSuper - 1) / kSuper, syn = (tiles_y + kSuper - 1) / kSuper, NS = sxn * syn;
     const int T = tiles_x * tiles_y;
     auto *k = reinterpret_cast<unsigned long long *>(super_keys);
@@ -1130,8 +1176,9 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
         launch_deep_tiles(s, T, tile_offsets, deep->len, deep->list, deep->count);
         (void)hipMemcpyAsync(deep->host_count, deep->count, sizeof(int), hipMemcpyDeviceToHost, s);
     }
-    hipLaunchKernelGGL(packed ? k_emit_tiles<true> : k_emit_tiles<false>, dim3(NS), dim3(kEmitThreads), 0, s, tiles_x,
-                       tiles_y, sxn, super_offsets, k, r2, tile_offsets, ids);
+    hipLaunchKernelGGL(packed ? k_emit_tiles<true> : k_emit_tiles<false>, dim3(8 + NS), dim3(kEmitThreads), 0, s,
+                       tiles_x, tiles_y, sxn, super_offsets, k, r2, tile_offsets, ids,
+                       std::max(1, num_isect / (4 * T)), tile_order);
     if (huge)
         hipLaunchKernelGGL(packed ? k_emit_chunks<true> : k_emit_chunks<false>, dim3(huge_grid), dim3(kEmitThreads), 0,
                            s, tiles_x, tiles_y, sxn, super_offsets, huge_list, huge_stats, chunk_base, chunk_counts, k,

@@ -72,12 +72,12 @@ __device__ __forceinline__ int load_batch(const float4 *__restrict__ rec, const 
 // seventh wave saves).
 template <bool LOG, bool FULL_OUT, bool COUNT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_raster_fwd(
-    int W, int H, int tiles_x, int T, const int *__restrict__ offsets, const int *__restrict__ ids,
-    const float4 *__restrict__ rec, const float4 *__restrict__ mrec, const float *__restrict__ bgp,
-    float *__restrict__ out_img, float *__restrict__ final_Ts, int *__restrict__ final_idx, float *__restrict__ out_depth,
+    int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets,
+    const int *__restrict__ ids, const float4 *__restrict__ rec, const float4 *__restrict__ mrec,
+    const float *__restrict__ bgp, float *__restrict__ out_img, float *__restrict__ final_Ts, int *__restrict__ final_idx, float *__restrict__ out_depth,
     float *__restrict__ out_normal, float *__restrict__ out_alpha, float *__restrict__ out_median,
     float *__restrict__ out_dist, unsigned long long *__restrict__ pair_counter, BlendLog blog, int deep_len) {
-    const int tile = xcd_strip_tile(blockIdx.x, tiles_x, T / tiles_x);
+    const int tile = order[blockIdx.x];
     if (tile < 0) return;
     __shared__ float4 s_rec[(FULL_OUT ? 6 : 5) * kThreads];  // the batch's records (load_batch planes)
     const int tx = tile % tiles_x, ty = tile / tiles_x;
@@ -284,16 +284,15 @@ constexpr unsigned long long kImgGrad = 0xfe0c0308d7654210ull;
 
 template <bool FULL>
 __global__ __launch_bounds__(kThreads) void k_raster_bwd(
-    int W, int H, int tiles_x, int T, const int *__restrict__ offsets, BlendLog blog, const float4 *__restrict__ rec,
+    int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets, BlendLog blog, const float4 *__restrict__ rec,
     const float *__restrict__ bgp, const float *__restrict__ final_Ts, const int *__restrict__ final_idx,
     const float *__restrict__ dL_dimg, const float *__restrict__ dL_ddepth, const float *__restrict__ dL_daccum,
     const float *__restrict__ dL_dnormal, const float *__restrict__ dL_dmedian, const float *__restrict__ dL_ddist,
-    float ddist_uniform, float *__restrict__ grads16, const int *__restrict__ tile_list, int deep_len) {
-    // tile_list: the deep tiles (their own launch); otherwise every other
-    // tile, XCD-mapped
-    const int tile = tile_list ? tile_list[blockIdx.x] : xcd_strip_tile(blockIdx.x, tiles_x, T / tiles_x);
+    float ddist_uniform, float *__restrict__ grads16, int deep_len) {
+    // order: every tile, or the deep tiles (their own launch)
+    const int tile = order[blockIdx.x];
     if (tile < 0) return;
-    if (!tile_list && offsets[tile + 1] - offsets[tile] >= deep_len) return;
+    if (offsets[tile + 1] - offsets[tile] >= deep_len) return;
     if (overflowed(blog)) return;  // an incomplete log: the step is redone with a larger pool
     constexpr int kWave = 64;
     // per wave: the staged entries' record planes (the image-only path
@@ -1002,13 +1001,12 @@ void launch_check_rcp(hipStream_t s, int efield, unsigned long long *bad) {
     hipLaunchKernelGGL(k_check_rcp, dim3((1u << 24) / 256), dim3(256), 0, s, (uint32_t)efield, bad);
 }
 
-void launch_raster_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *offsets, const int *ids,
+void launch_raster_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets, const int *ids,
                        const float *rec, const float *mrec, const float *bg, float *out_img, float *final_Ts, int *final_idx,
                        float *out_depth, float *out_normal, float *out_alpha, float *out_median, float *out_dist,
                        unsigned long long *pair_counter, const BlendLog *blog, bool full_outputs,
                        const DeepTiles &deep) {
-    const int T = tiles_x * tiles_y;
-    const int grid = xcd_strip_grid(tiles_x, tiles_y);
+    const int grid = tile_order_ints(tiles_x, tiles_y);
     const BlendLog lg = blog ? *blog : BlendLog{};
     const int deep_len = deep.n > 0 ? deep.len : INT32_MAX;
     if (deep.n > 0) {
@@ -1036,7 +1034,7 @@ void launch_raster_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, co
         if (!defer) (void)hipEventRecord(deep.join, sd);
     }
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), 0, s, W, H, tiles_x, T, offsets, ids,
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), 0, s, W, H, tiles_x, order, offsets, ids,
                            reinterpret_cast<const float4 *>(rec), reinterpret_cast<const float4 *>(mrec), bg,
                            out_img, final_Ts, final_idx, out_depth,
                            out_normal, out_alpha, out_median, out_dist, pair_counter, lg, deep_len);
@@ -1062,26 +1060,25 @@ void launch_deep_tiles(hipStream_t s, int T, const int *offsets, int deep_len, i
 
 int64_t deep_pixel_entries(int n_deep) { return (int64_t)n_deep * 256 * kDeepMaxBlend; }
 
-bool launch_raster_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *offsets,
+bool launch_raster_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets,
                        const BlendLog &blog, const float *rec,
                        const float *bg, const float *final_Ts, const int *final_idx, const float *dL_dimg,
                        const float *dL_ddepth, const float *dL_daccum, const float *dL_dnormal,
                        const float *dL_dmedian, const float *dL_ddist, float ddist_uniform, float *grads16,
                        const DeepTiles &deep) {
-    const int T = tiles_x * tiles_y;
-    const int grid = xcd_strip_grid(tiles_x, tiles_y);
+    const int grid = tile_order_ints(tiles_x, tiles_y);
     const bool full = dL_ddepth || dL_daccum || dL_dnormal || dL_dmedian || dL_ddist || ddist_uniform != 0.0f;
     auto launch = [&](hipStream_t st, int blocks, const int *list, int deep_len) {
         if (full)
-            hipLaunchKernelGGL(k_raster_bwd<true>, dim3(blocks), dim3(kThreads), 0, st, W, H, tiles_x, T, offsets, blog,
+            hipLaunchKernelGGL(k_raster_bwd<true>, dim3(blocks), dim3(kThreads), 0, st, W, H, tiles_x, list, offsets, blog,
                                reinterpret_cast<const float4 *>(rec), bg, final_Ts, final_idx,
                                dL_dimg, dL_ddepth, dL_daccum, dL_dnormal, dL_dmedian, dL_ddist, ddist_uniform,
-                               grads16, list, deep_len);
+                               grads16, deep_len);
         else
-            hipLaunchKernelGGL(k_raster_bwd<false>, dim3(blocks), dim3(kThreads), 0, st, W, H, tiles_x, T, offsets,
+            hipLaunchKernelGGL(k_raster_bwd<false>, dim3(blocks), dim3(kThreads), 0, st, W, H, tiles_x, list, offsets,
                                blog, reinterpret_cast<const float4 *>(rec), bg, final_Ts, final_idx,
                                dL_dimg, dL_ddepth, dL_daccum, dL_dnormal, dL_dmedian, dL_ddist, ddist_uniform,
-                               grads16, list, deep_len);
+                               grads16, deep_len);
     };
     if (deep.n > 0) {
         // the deep tiles' long log replays start at once, on their own
@@ -1091,12 +1088,12 @@ bool launch_raster_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, co
         (void)hipStreamWaitEvent(s, deep.logged, 0);
         (void)hipEventRecord(deep.fork, s);
         (void)hipStreamWaitEvent(deep.stream, deep.fork, 0);
-        launch(deep.stream, deep.n, deep.list, 0);
+        launch(deep.stream, deep.n, deep.list, INT32_MAX);
         (void)hipEventRecord(deep.join, deep.stream);
-        launch(s, grid, nullptr, deep.len);
+        launch(s, grid, order, deep.len);
         (void)hipStreamWaitEvent(s, deep.join, 0);
     } else {
-        launch(s, grid, nullptr, INT32_MAX);
+        launch(s, grid, order, INT32_MAX);
     }
     return !full;
 }

@@ -48,14 +48,15 @@ __device__ __forceinline__ int load_batch3(const float4 *__restrict__ rec, const
 // BlendLog).
 // Outputs: out_img and final_Ts[.][0] (the transmittance).
 template <bool LOG>
-__global__ __launch_bounds__(kThreads) void k_raster3d_fwd(int W, int H, int tiles_x, int T,
+__global__ __launch_bounds__(kThreads) void k_raster3d_fwd(int W, int H, int tiles_x,
+                                                           const int *__restrict__ order,
                                                            const int *__restrict__ offsets,
                                                            const int *__restrict__ ids,
                                                            const float4 *__restrict__ rec,
                                                            const float4 *__restrict__ boxes,
                                                            const float *__restrict__ bgp, float *__restrict__ out_img,
                                                            float *__restrict__ final_Ts, BlendLog blog) {
-    const int tile = xcd_strip_tile(blockIdx.x, tiles_x, T / tiles_x);
+    const int tile = order[blockIdx.x];
     if (tile < 0) return;
     __shared__ float4 s_rec[3 * kThreads];
     __shared__ unsigned char s_list[4][kThreads];
@@ -149,7 +150,8 @@ __global__ __launch_bounds__(kThreads) void k_raster3d_fwd(int W, int H, int til
 // The log arrives as separate read-only, non-aliasing pointers (not the
 // BlendLog struct) so that the compiler can load the wave-uniform entries
 // with scalar loads beside the loop's gradient atomics.
-__global__ __launch_bounds__(kThreads) void k_raster3d_bwd(int W, int H, int tiles_x, int T,
+__global__ __launch_bounds__(kThreads) void k_raster3d_bwd(int W, int H, int tiles_x,
+                                                           const int *__restrict__ order,
                                                            const int *__restrict__ offsets,
                                                            const uint4 *__restrict__ log_ent,
                                                            const float *__restrict__ log_ckpt,
@@ -161,7 +163,7 @@ __global__ __launch_bounds__(kThreads) void k_raster3d_bwd(int W, int H, int til
                                                            const float *__restrict__ final_Ts,
                                                            const float *__restrict__ dL_dimg,
                                                            float *__restrict__ grads16) {
-    const int tile = xcd_strip_tile(blockIdx.x, tiles_x, T / tiles_x);
+    const int tile = order[blockIdx.x];
     if (tile < 0) return;
     if (*log_overflow) return;  // an incomplete log: the step is redone with a larger pool
     constexpr int kWave = 64;
@@ -252,29 +254,27 @@ __global__ __launch_bounds__(kThreads) void k_raster3d_bwd(int W, int H, int til
 
 namespace mskern {
 
-void launch_raster3d_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *offsets, const int *ids,
+void launch_raster3d_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets, const int *ids,
                          const float *rec, const float *boxes, const float *bg, float *out_img, float *final_Ts,
                          const BlendLog *blog) {
-    const int T = tiles_x * tiles_y;
-    if (T <= 0) return;
-    const int grid = xcd_strip_grid(tiles_x, tiles_y);
+    if (tiles_x * tiles_y <= 0) return;
+    const int grid = tile_order_ints(tiles_x, tiles_y);
     const auto *r4 = reinterpret_cast<const float4 *>(rec);
     const auto *b4 = reinterpret_cast<const float4 *>(boxes);
     if (blog)
-        hipLaunchKernelGGL(k_raster3d_fwd<true>, dim3(grid), dim3(kThreads), 0, s, W, H, tiles_x, T, offsets, ids,
+        hipLaunchKernelGGL(k_raster3d_fwd<true>, dim3(grid), dim3(kThreads), 0, s, W, H, tiles_x, order, offsets, ids,
                            r4, b4, bg, out_img, final_Ts, *blog);
     else
-        hipLaunchKernelGGL(k_raster3d_fwd<false>, dim3(grid), dim3(kThreads), 0, s, W, H, tiles_x, T, offsets, ids,
+        hipLaunchKernelGGL(k_raster3d_fwd<false>, dim3(grid), dim3(kThreads), 0, s, W, H, tiles_x, order, offsets, ids,
                            r4, b4, bg, out_img, final_Ts, BlendLog{});
 }
 
-void launch_raster3d_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *offsets,
+void launch_raster3d_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets,
                          const BlendLog &blog, const float *rec, const float *bg, const float *final_Ts,
                          const float *dL_dimg, float *grads16) {
-    const int T = tiles_x * tiles_y;
-    if (T <= 0) return;
-    const int grid = xcd_strip_grid(tiles_x, tiles_y);
-    hipLaunchKernelGGL(k_raster3d_bwd, dim3(grid), dim3(kThreads), 0, s, W, H, tiles_x, T, offsets, blog.ent,
+    if (tiles_x * tiles_y <= 0) return;
+    const int grid = tile_order_ints(tiles_x, tiles_y);
+    hipLaunchKernelGGL(k_raster3d_bwd, dim3(grid), dim3(kThreads), 0, s, W, H, tiles_x, order, offsets, blog.ent,
                        blog.ckpt, blog.table, blog.wave_cnt, blog.overflow, reinterpret_cast<const float4 *>(rec), bg,
                        final_Ts, dL_dimg, grads16);
 }

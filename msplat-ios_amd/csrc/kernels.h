@@ -67,7 +67,9 @@ constexpr int kBinMaxBlocks = 256;
 // lists need super_keys_tmp (the size of super_keys), huge_list[NS],
 // huge_stats[2] (zero on entry), chunk_base[NS], merge_base[NS] and
 // chunk_counts[huge_chunk_ints(total, NS)], and super_stats[3] receives
-// their merge-tile count.  total_keys = the pair count (super_stats[0]).
+// their merge-tile count.  total_keys = the pair count (super_stats[0]),
+// num_isect = the intersection count.  tile_order (tile_order_ints) receives
+// the order the rasterizers take the tiles in.
 // The deep-tile scan launch_bin_tiles queues once the tile offsets exist
 // (before the emission kernels): the tiles with at least `len` entries into
 // `list`, their number into *count, copied to *host_count.
@@ -80,7 +82,9 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
                       uint64_t *super_keys, uint64_t *super_keys_tmp, int *super_stats, int *huge_list,
                       int *huge_stats, int *chunk_base, int *chunk_counts, int *merge_base, int total_keys,
                       int *tile_counts, int *tile_offsets, int *tile_stats, int *tile_temp, int *ids,
-                      bool force_wide_keys, const DeepScan *deep = nullptr);
+                      int num_isect, int *tile_order, bool force_wide_keys, const DeepScan *deep = nullptr);
+// Ints of tile_order: the rasterizers' workgroups, each with its tile (or -1).
+int tile_order_ints(int tiles_x, int tiles_y);
 constexpr int kSuperTile = 4;
 // Keys of a super-tile list that one workgroup sorts in LDS, and keys per
 // counting and emission unit of a longer (huge) list.
@@ -127,14 +131,15 @@ struct DeepTiles {
 };
 void launch_deep_tiles(hipStream_t s, int T, const int *offsets, int deep_len, int *deep_list, int *count);
 int64_t deep_pixel_entries(int n_deep);
-void launch_raster_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *offsets, const int *ids,
+void launch_raster_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets,
+                       const int *ids,
                        const float *rec, const float *mrec, const float *bg, float *out_img, float *final_Ts, int *final_idx,
                        float *out_depth, float *out_normal, float *out_alpha, float *out_median, float *out_dist,
                        unsigned long long *pair_counter, const msr::BlendLog *blog, bool full_outputs,
                        const DeepTiles &deep);
 // Returns true when the image-only kernel ran: grads16 then holds its sums
 // (launch_finish_image_grads / launch_project_bwd finish them).
-bool launch_raster_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *offsets,
+bool launch_raster_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets,
                        const msr::BlendLog &blog, const float *rec,
                        const float *bg, const float *final_Ts, const int *final_idx, const float *dL_dimg,
                        const float *dL_ddepth, const float *dL_daccum, const float *dL_dnormal,
@@ -146,10 +151,11 @@ constexpr int kBlendLogEntryBytes = 16;
 // boxes = their quadrant-mask boxes.  blend_log / t_ckpt / wave_cnt as for
 // launch_raster_fwd (nullptr: render only).  The backward adds the per-splat
 // sums to grads16 (launch_finish3d_grads finishes them).
-void launch_raster3d_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *offsets, const int *ids,
+void launch_raster3d_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets,
+                         const int *ids,
                          const float *rec, const float *boxes, const float *bg, float *out_img, float *final_Ts,
                          const msr::BlendLog *blog);
-void launch_raster3d_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *offsets,
+void launch_raster3d_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets,
                          const msr::BlendLog &blog, const float *rec, const float *bg, const float *final_Ts,
                          const float *dL_dimg, float *grads16);
 // Adds to *bad the number of floats of exponent field efield (1..254, both
