@@ -14,6 +14,7 @@
 #include <exception>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "kernels.h"
@@ -52,6 +53,10 @@ enum StageId { ST_PROJECT, ST_SCAN, ST_SCATTER_SORT, ST_RASTER_FWD, ST_LOSS, ST_
 const char *kStageNames[ST_COUNT] = {"project_fwd", "tile_scan", "scatter_sort", "raster_fwd",
                                      "ssim_l1",     "raster_bwd", "project_bwd_adam"};
 
+// Published slots: the super-tile scan, the deep tiles, the training step.
+enum PubSlot { PUB_SUPER, PUB_DEEP, PUB_STEP, PUB_COUNT };
+constexpr int kPubInts = 512;  // two doubles and at most 258 counters, and the flag
+
 constexpr size_t kD2HChunk = size_t(8) << 20;  // bytes per pinned download chunk
 
 // Deep-tile threshold: no tile of the 500k and 3M-splat blob workloads holds
@@ -71,6 +76,10 @@ struct Engine {
     int *pinned_i = nullptr;     // small pinned readback area
     int *pinned_ctr = nullptr;   // the blend-log pool's counters
     double *pinned_d = nullptr;
+    // what kernels publish (mskern::Publish): per slot kPubInts ints, the
+    // last of them the flag
+    int *pub = nullptr;
+    int pub_seq = 0;
     // two pinned chunks of kD2HChunk bytes for large downloads (RGBA8
     // frames) and the events of their DMAs
     unsigned char *stage = nullptr;
@@ -140,7 +149,7 @@ struct Engine {
     double log_fill[2] = {0.0, 0.0};
     msr::BlendLog log_desc{};  // the current frame's pool layout
     hipStream_t deep_stream = nullptr;  // default priority, non-blocking
-    hipEvent_t deep_fork = nullptr, deep_join = nullptr, deep_logged = nullptr;
+    hipEvent_t deep_fork = nullptr, deep_started = nullptr, deep_join = nullptr, deep_logged = nullptr;
     hipEvent_t ev[ST_COUNT + 1] = {};
     float stage_ms[ST_COUNT] = {};
     bool stage_valid[ST_COUNT] = {};
@@ -201,6 +210,35 @@ float *mask_recs() { return P<float>(g_eng.rec) + (size_t)g_eng.n * MSPLAT_REC_F
 
 int check_rcp_locked(int lo, int hi, int64_t *bad);
 
+// A new publication into a slot, and the wait for it: the flag arrives as
+// soon as the kernel that publishes has run, while a copy and a stream
+// synchronisation also wait for what is queued behind it and cost two trips
+// through the runtime (14.8 against 9.7 us for an empty kernel).  Ends when
+// the stream has drained or failed without the flag.
+mskern::Publish publish_to(PubSlot slot) {
+    Engine &E = g_eng;
+    E.pub_seq = E.pub_seq == INT_MAX ? 1 : E.pub_seq + 1;
+    int *p = E.pub + (size_t)slot * kPubInts;
+    return {p, p + kPubInts - 1, E.pub_seq};
+}
+int wait_published(const mskern::Publish &p) {
+    const auto there = [&] { return __atomic_load_n(p.flag, __ATOMIC_ACQUIRE) == p.seq; };
+    for (unsigned spin = 1; !there(); ++spin) {
+        __builtin_ia32_pause();
+        if (spin % 4096) continue;
+        const hipError_t e = hipStreamQuery(g_eng.stream);
+        if (e == hipErrorNotReady) {
+            std::this_thread::yield();
+            continue;
+        }
+        HIPC(e);
+        if (there()) break;
+        set_err("a kernel ended without its result");
+        return MSPLAT_E_HIP;
+    }
+    return MSPLAT_OK;
+}
+
 int init_locked() {
     if (g_eng.ready) return MSPLAT_OK;
     int count = 0;
@@ -224,6 +262,8 @@ int init_locked() {
     HIPC(hipHostMalloc((void **)&g_eng.pinned_i, 64 * sizeof(int), hipHostMallocDefault));
     HIPC(hipHostMalloc((void **)&g_eng.pinned_ctr, 264 * sizeof(int), hipHostMallocDefault));
     HIPC(hipHostMalloc((void **)&g_eng.pinned_d, 16 * sizeof(double), hipHostMallocDefault));
+    HIPC(hipHostMalloc((void **)&g_eng.pub, PUB_COUNT * kPubInts * sizeof(int), hipHostMallocCoherent));
+    std::memset(g_eng.pub, 0, PUB_COUNT * kPubInts * sizeof(int));
     HIPC(hipHostMalloc((void **)&g_eng.stage, 2 * kD2HChunk, hipHostMallocDefault));
     for (auto &e : g_eng.stage_ev) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     for (int i = 0; i <= ST_COUNT; ++i) HIPC(hipEventCreate(&g_eng.ev[i]));
@@ -322,6 +362,7 @@ int deep_tiles(mskern::DeepTiles &deep) {
     if (!E.deep_stream) {
         HIPC(hipStreamCreateWithFlags(&E.deep_stream, hipStreamNonBlocking));
         HIPC(hipEventCreateWithFlags(&E.deep_fork, hipEventDisableTiming));
+        HIPC(hipEventCreateWithFlags(&E.deep_started, hipEventDisableTiming));
         HIPC(hipEventCreateWithFlags(&E.deep_join, hipEventDisableTiming));
         HIPC(hipEventCreateWithFlags(&E.deep_logged, hipEventDisableTiming));
     }
@@ -330,6 +371,7 @@ int deep_tiles(mskern::DeepTiles &deep) {
     deep.list = P<int>(E.deep_list);
     deep.stream = E.deep_stream;
     deep.fork = E.deep_fork;
+    deep.started = E.deep_started;
     deep.join = E.deep_join;
     deep.logged = E.deep_logged;
     return MSPLAT_OK;
@@ -396,19 +438,15 @@ int plan_log_pool(msr::BlendLog &L) {
     return MSPLAT_OK;
 }
 
-// Queues the copy of the pool's counters and overflow flag after a logging
-// forward; once the stream has synchronised, log_account returns whether
-// the log overflowed and, if not, records the frame's demand (each claim is
-// counted in its sub-pool's counter, also when the spill region served it).
-int log_readback(const msr::BlendLog &L, hipStream_t s) {
-    HIPC(hipMemcpyAsync(g_eng.pinned_ctr, L.counters, (size_t)(L.nsub + 2) * 4, hipMemcpyDeviceToHost, s));
-    return MSPLAT_OK;
-}
-bool log_account(const msr::BlendLog &L) {
+// Reads the pool's counters and overflow flag, once they are on the host:
+// whether the log overflowed and, if not, records the frame's demand (each
+// claim is counted in its sub-pool's counter, also when the spill region
+// served it).
+bool log_account(const msr::BlendLog &L, const int *ctr) {
     Engine &E = g_eng;
-    if (g_eng.pinned_ctr[L.nsub + 1] != 0) return true;
+    if (ctr[L.nsub + 1] != 0) return true;
     int64_t demand = 0;
-    for (int i = 0; i < L.nsub; ++i) demand += g_eng.pinned_ctr[i];
+    for (int i = 0; i < L.nsub; ++i) demand += ctr[i];
     E.log_demand = demand;
     double &fill = E.log_fill[E.gs3d];
     fill = std::max(fill, (double)demand / (double)log_static_estimate(E));
@@ -430,7 +468,8 @@ void grow_log_pool() {
     ++E.log_redos;
 }
 
-int raster_fwd_locked(bool log, bool full) {
+// cleared: the log's counters are zero already.
+int raster_fwd_locked(bool log, bool full, bool cleared = false) {
     Engine &E = g_eng;
     msr::BlendLog blog{};
     mskern::DeepTiles deep;
@@ -448,7 +487,7 @@ int raster_fwd_locked(bool log, bool full) {
     }
     if (log) {
         CHECK(plan_log_pool(blog));
-        CHECK(reset_log_pool(blog));
+        if (!cleared) CHECK(reset_log_pool(blog));
     }
     deep.defer_log = log && E.defer_deep_log;
     if (E.gs3d) {
@@ -480,9 +519,10 @@ int log_forward_checked(bool full) {
     Engine &E = g_eng;
     for (;;) {
         CHECK(raster_fwd_locked(true, full));
-        CHECK(log_readback(E.log_desc, E.stream));
+        HIPC(hipMemcpyAsync(E.pinned_ctr, E.log_desc.counters, (size_t)(E.log_desc.nsub + 2) * 4,
+                            hipMemcpyDeviceToHost, E.stream));
         HIPC(hipStreamSynchronize(E.stream));
-        if (!log_account(E.log_desc)) return MSPLAT_OK;
+        if (!log_account(E.log_desc, E.pinned_ctr)) return MSPLAT_OK;
         grow_log_pool();
     }
 }
@@ -545,7 +585,9 @@ int forward_locked(const MsplatCamera *cam, const MsplatGaussians *g, const floa
     for (int i = 0; i < ST_COUNT; ++i) E.stage_valid[i] = false;
 
     stage_mark(ST_PROJECT);
-    HIPC(hipMemsetAsync(E.stats.p, 0, 64, s));
+    const int log_ints = log ? log_subpools(T) + 2 : 0;
+    if (log) CHECK(ensure(E.log_ctr, (size_t)log_ints * 4));
+    mskern::launch_zero_counters(s, P<int>(E.stats), 16, P<int>(E.log_ctr), log_ints);
     if (E.count_pairs) HIPC(hipMemsetAsync(E.pair_counter.p, 0, 40, s));
     // the 3DGS rasterizers count nothing: no counters for this forward
     if (gs3d) std::fill(E.pairs, E.pairs + 5, int64_t(0));
@@ -558,14 +600,16 @@ int forward_locked(const MsplatCamera *cam, const MsplatGaussians *g, const floa
                                    P<uint32_t>(E.rect), reinterpret_cast<unsigned long long *>(P<int>(E.stats) + 8),
                                    nullptr);
     stage_mark(ST_SCAN);
+    const mskern::Publish counted = publish_to(PUB_SUPER);
     mskern::launch_super_count(s, N, cam->tiles_x, cam->tiles_y, P<int>(E.radii), P<uint32_t>(E.rect),
                                P<int>(E.super_counts), P<int>(E.super_offsets), P<int>(E.super_cm),
-                               P<int>(E.stats) + 4, P<int>(E.super_tmp));
-    HIPC(hipMemcpyAsync(E.pinned_i, E.stats.p, 16 * sizeof(int), hipMemcpyDeviceToHost, s));
-    HIPC(hipStreamSynchronize(s));
+                               P<int>(E.stats) + 4, P<int>(E.super_tmp),
+                               reinterpret_cast<const unsigned long long *>(P<int>(E.stats) + 8), counted);
+    HIPC(hipGetLastError());
+    CHECK(wait_published(counted));
     unsigned long long isect64;
-    std::memcpy(&isect64, E.pinned_i + 8, sizeof(isect64));
-    const int S_total = E.pinned_i[4], super_max = E.pinned_i[5];
+    std::memcpy(&isect64, counted.data, sizeof(isect64));
+    const int S_total = counted.data[2], super_max = counted.data[3];
     if (isect64 > 0x7fffffffull || S_total < 0) {
         set_err("tile intersection count %llu overflows int32", isect64);
         return MSPLAT_E_CAPACITY;
@@ -593,7 +637,7 @@ int forward_locked(const MsplatCamera *cam, const MsplatGaussians *g, const floa
         dscan.len = E.deep_frame;
         dscan.list = P<int>(E.deep_list);
         dscan.count = P<int>(E.stats) + 14;
-        dscan.host_count = E.pinned_i + 14;
+        dscan.out = publish_to(PUB_DEEP);
     }
     mskern::launch_bin_tiles(s, N, cam->tiles_x, cam->tiles_y, P<int>(E.radii), P<uint32_t>(E.rect),
                              P<float>(E.depths), P<int>(E.super_offsets), P<int>(E.super_cm), super_max,
@@ -603,11 +647,12 @@ int forward_locked(const MsplatCamera *cam, const MsplatGaussians *g, const floa
                              P<int>(E.scan_tmp), P<int>(E.ids), I, P<int>(E.tile_order), E.wide_keys, scan_deep ? &dscan : nullptr);
     E.n_deep = 0;
     if (scan_deep) {
-        HIPC(hipStreamSynchronize(s));
-        E.n_deep = E.pinned_i[14];
+        HIPC(hipGetLastError());
+        CHECK(wait_published(dscan.out));
+        E.n_deep = dscan.out.data[0];
     }
     stage_mark(ST_RASTER_FWD);
-    CHECK(raster_fwd_locked(log, full));
+    CHECK(raster_fwd_locked(log, full, true));
     HIPC(hipGetLastError());
     return MSPLAT_OK;
 }
@@ -1112,7 +1157,6 @@ static int train_step_once(const MsplatCamera *cam, const MsplatGaussians *g, co
     CHECK(ensure(E.dL_dimg, Pn * 12));
     CHECK(loss_locked(W, H, P<float>(E.out_img), gt, lambda_dist != 0.f ? P<float>(E.out_dist) : nullptr,
                       lambda_l1, lambda_dist, lambda_dssim, P<float>(E.dL_dimg)));
-    HIPC(hipMemcpyAsync(E.pinned_d, E.loss.p, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
     stage_mark(ST_RASTER_BWD);
     CHECK(ensure(E.grads16, (size_t)N * 64));
     mskern::launch_zero16(s, P<float>(E.grads16), (int64_t)N * 4);
@@ -1148,20 +1192,25 @@ static int train_step_once(const MsplatCamera *cam, const MsplatGaussians *g, co
     E.raster_grads = true;
     E.g16_moments = t_moments;
     stage_mark(ST_COUNT);
-    CHECK(log_readback(blog, s));
+    const mskern::Publish done = publish_to(PUB_STEP);
+    mskern::launch_step_report(s, P<double>(E.loss), blog.counters, blog.nsub + 2, done);
     HIPC(hipGetLastError());
-    HIPC(hipStreamSynchronize(s));
-    *log_overflow = log_account(blog);
+    // behind the whole step in stream order
+    CHECK(wait_published(done));
+    *log_overflow = log_account(blog, done.data + 4);
     if (*log_overflow) {
         E.have_grads = E.raster_grads = false;
         return MSPLAT_OK;
     }
-    if (loss_host) *loss_host = (float)E.pinned_d[0];
+    double loss;
+    std::memcpy(&loss, done.data, sizeof(loss));
+    if (loss_host) *loss_host = (float)loss;
     if (E.count_pairs) {
         HIPC(hipMemcpyAsync(E.pairs, E.pair_counter.p, 40, hipMemcpyDeviceToHost, s));
         HIPC(hipStreamSynchronize(s));
     }
     if (E.timing) {
+        HIPC(hipStreamSynchronize(s));
         for (int i = 0; i < ST_COUNT; ++i) {
             HIPC(hipEventElapsedTime(&E.stage_ms[i], E.ev[i], E.ev[i + 1]));
             E.stage_valid[i] = true;
@@ -1221,7 +1270,6 @@ static int train_step3d_once(const MsplatCamera *cam, const MsplatGaussians *g, 
     stage_mark(ST_LOSS);
     CHECK(ensure(E.dL_dimg, Pn * 12));
     CHECK(loss_locked(W, H, P<float>(E.out_img), gt, nullptr, lambda_l1, 0.f, lambda_dssim, P<float>(E.dL_dimg)));
-    HIPC(hipMemcpyAsync(E.pinned_d, E.loss.p, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
     stage_mark(ST_RASTER_BWD);
     CHECK(ensure(E.grads16, (size_t)N * 64));
     mskern::launch_zero16(s, P<float>(E.grads16), (int64_t)N * 4);
@@ -1251,16 +1299,21 @@ static int train_step3d_once(const MsplatCamera *cam, const MsplatGaussians *g, 
     E.raster_grads = true;
     E.g16_moments = true;
     stage_mark(ST_COUNT);
-    CHECK(log_readback(blog, s));
+    const mskern::Publish done = publish_to(PUB_STEP);
+    mskern::launch_step_report(s, P<double>(E.loss), blog.counters, blog.nsub + 2, done);
     HIPC(hipGetLastError());
-    HIPC(hipStreamSynchronize(s));
-    *log_overflow = log_account(blog);
+    // behind the whole step in stream order
+    CHECK(wait_published(done));
+    *log_overflow = log_account(blog, done.data + 4);
     if (*log_overflow) {
         E.have_grads = E.raster_grads = false;
         return MSPLAT_OK;
     }
-    if (loss_host) *loss_host = (float)E.pinned_d[0];
+    double loss;
+    std::memcpy(&loss, done.data, sizeof(loss));
+    if (loss_host) *loss_host = (float)loss;
     if (E.timing) {
+        HIPC(hipStreamSynchronize(s));
         for (int i = 0; i < ST_COUNT; ++i) {
             HIPC(hipEventElapsedTime(&E.stage_ms[i], E.ev[i], E.ev[i + 1]));
             E.stage_valid[i] = true;

@@ -139,18 +139,35 @@ __global__ __launch_bounds__(1024) void k_off_totals(int nb, int *__restrict__ t
     if (threadIdx.x == 0) stats[0] = all;
 }
 
-__global__ __launch_bounds__(kScanT) void k_off_add(int T, int *__restrict__ offsets, int *__restrict__ cursor,
+__global__ __launch_bounds__(kScanT) void k_off_add(int T, int *__restrict__ offsets,
                                                     const int *__restrict__ totals, const int *__restrict__ stats) {
     const int base = blockIdx.x * kScanChunk + threadIdx.x * kScanI;
     const int o = totals[blockIdx.x];
 #pragma unroll
     for (int k = 0; k < kScanI; ++k)
-        if (base + k < T) {
-            const int v = offsets[base + k] + o;
-            offsets[base + k] = v;
-            if (cursor) cursor[base + k] = v;
-        }
+        if (base + k < T) offsets[base + k] += o;
     if (blockIdx.x == 0 && threadIdx.x == 0) offsets[T] = stats[0];
+}
+
+// What a scan leaves for the host and the deep tiles it lists.
+struct ScanExtra {
+    mskern::Publish out;                         // the scan's results (data null: none)
+    const unsigned long long *isect = nullptr;   // set: out = {*isect, total, largest}
+    int deep_len = 0;                            // > 0: out = {deep tiles}, listed
+    int *deep_list = nullptr, *deep_count = nullptr;
+};
+__device__ __forceinline__ void publish(const mskern::Publish &out, const int *v, int n) {
+    for (int k = 0; k < n; ++k) out.data[k] = v[k];
+    __hip_atomic_store(out.flag, out.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void publish_scan(const ScanExtra &x, int total, int largest, int deep) {
+    if (x.isect) {
+        const unsigned long long q = *x.isect;
+        const int v[4] = {(int)(uint32_t)q, (int)(q >> 32), total, largest};
+        publish(x.out, v, 4);
+    } else {
+        publish(x.out, &deep, 1);
+    }
 }
 
 // The same scan in one workgroup of 1024 threads, for counts[] short enough
@@ -160,11 +177,12 @@ constexpr int kScanSmallT = 1024, kScanSmallChunk = kScanSmallT * kScanI;
 constexpr int kScanSmallMax = 4 * kScanSmallChunk;  // at most 4 rounds
 
 __global__ __launch_bounds__(kScanSmallT) void k_scan_small(int T, const int *__restrict__ counts,
-                                                            int *__restrict__ offsets, int *__restrict__ cursor,
-                                                            int *__restrict__ stats) {
-    __shared__ int s_w[kScanSmallT / 64];
+                                                            int *__restrict__ offsets, int *__restrict__ stats,
+                                                            ScanExtra x) {
+    __shared__ int s_w[kScanSmallT / 64], s_mx[kScanSmallT / 64], s_deep;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int carry = 0, mx = 0;
+    if (threadIdx.x == 0) s_deep = 0;
     for (int base = 0; base < T; base += kScanSmallChunk) {
         const int i0 = base + (int)threadIdx.x * kScanI;
         int v[kScanI], sum = 0;
@@ -194,18 +212,28 @@ __global__ __launch_bounds__(kScanSmallT) void k_scan_small(int T, const int *__
         for (int k = 0; k < kScanI; ++k)
             if (i0 + k < T) {
                 offsets[i0 + k] = run;
-                if (cursor) cursor[i0 + k] = run;
                 run += v[k];
+                if (x.deep_len > 0 && v[k] >= x.deep_len) x.deep_list[atomicAdd(&s_deep, 1)] = i0 + k;
             }
         carry += tot;
     }
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) mx = max(mx, __shfl_xor(mx, d, 64));
-    if (lane == 0 && mx > 0) atomicMax(&stats[1], mx);
+    if (lane == 0) s_mx[wave] = mx;
+    __syncthreads();
     if (threadIdx.x == 0) {
+        for (int w = 1; w < kScanSmallT / 64; ++w) mx = max(mx, s_mx[w]);
         stats[0] = carry;
+        stats[1] = mx;
         offsets[T] = carry;
+        if (x.deep_len > 0) *x.deep_count = s_deep;
+        if (x.out.data) publish_scan(x, carry, mx, s_deep);
     }
+}
+
+// The publication of a scan that took three kernels.
+__global__ void k_publish_scan(const int *__restrict__ stats, ScanExtra x) {
+    publish_scan(x, stats[0], stats[1], x.deep_len > 0 ? *x.deep_count : 0);
 }
 
 // ---- super-tile histogram and scatter -------------------------------------
@@ -1072,18 +1100,20 @@ int tile_order_ints(int tiles_x, int tiles_y) { return msd::xcd_strip_grid(tiles
 
 int64_t tile_scan_temp_ints(int T) { return (T + kScanChunk - 1) / kScanChunk + 1; }
 
-// Exclusive scan of counts[T] into offsets[T + 1] (and cursor[T] if given);
-// stats[0] = total, stats[1] = max(stats[1], largest count).
-static void launch_scan_counts(hipStream_t s, int T, const int *counts, int *offsets, int *cursor, int *stats,
-                               int *temp) {
+// Exclusive scan of counts[T] into offsets[T + 1]; stats[0] = total, stats[1]
+// = the largest count (zero on entry).
+static void launch_scan_counts(hipStream_t s, int T, const int *counts, int *offsets, int *stats, int *temp,
+                               const ScanExtra &x) {
     if (T <= kScanSmallMax) {
-        hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kScanSmallT), 0, s, T, counts, offsets, cursor, stats);
+        hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kScanSmallT), 0, s, T, counts, offsets, stats, x);
         return;
     }
     const int nb = (T + kScanChunk - 1) / kScanChunk;
     hipLaunchKernelGGL(k_off_local, dim3(nb), dim3(kScanT), 0, s, T, counts, offsets, temp, stats);
     hipLaunchKernelGGL(k_off_totals, dim3(1), dim3(1024), 0, s, nb, temp, stats);
-    hipLaunchKernelGGL(k_off_add, dim3(nb), dim3(kScanT), 0, s, T, offsets, cursor, temp, stats);
+    hipLaunchKernelGGL(k_off_add, dim3(nb), dim3(kScanT), 0, s, T, offsets, temp, stats);
+    if (x.deep_len > 0) launch_deep_tiles(s, T, offsets, x.deep_len, x.deep_list, x.deep_count);
+    if (x.out.data) hipLaunchKernelGGL(k_publish_scan, dim3(1), dim3(1), 0, s, stats, x);
 }
 
 static void bin_chunks(int n, int *blocks, int *chunk) {
@@ -1092,7 +1122,8 @@ static void bin_chunks(int n, int *blocks, int *chunk) {
 }
 
 void launch_super_count(hipStream_t s, int n, int tiles_x, int tiles_y, const int *radii, const uint32_t *rect,
-                        int *super_counts, int *super_offsets, int *super_cm, int *super_stats, int *temp) {
+                        int *super_counts, int *super_offsets, int *super_cm, int *super_stats, int *temp,
+                        const unsigned long long *isect, const Publish &out) {
     const int sxn = (tiles_x + kSuper - 1) / kSuper, syn = (tiles_y + kSuper - 1) / kSuper, NS = sxn * syn;
     int blocks, chunk;
     bin_chunks(n, &blocks, &chunk);
@@ -1102,7 +1133,10 @@ void launch_super_count(hipStream_t s, int n, int tiles_x, int tiles_y, const in
     // with no splats the matrix has no rows and every count is zero
     hipLaunchKernelGGL(k_super_cols, dim3((NS + kColW - 1) / kColW), dim3(kColW * kColWaves), 0, s,
                        n > 0 ? blocks : 0, NS, super_cm, super_counts);
-    launch_scan_counts(s, NS, super_counts, super_offsets, nullptr, super_stats, temp);
+    ScanExtra x;
+    x.out = out;
+    x.isect = isect;
+    launch_scan_counts(s, NS, super_counts, super_offsets, super_stats, temp, x);
 }
 
 void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int *radii, const uint32_t *rect,
@@ -1171,11 +1205,14 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
                            tiles_x, tiles_y, sxn, super_offsets, huge_list, huge_stats, chunk_base, k, kt, r2,
                            chunk_counts, tile_counts);
     }
-    launch_scan_counts(s, T, tile_counts, tile_offsets, nullptr, tile_stats, tile_temp);
+    ScanExtra x;
     if (deep) {
-        launch_deep_tiles(s, T, tile_offsets, deep->len, deep->list, deep->count);
-        (void)hipMemcpyAsync(deep->host_count, deep->count, sizeof(int), hipMemcpyDeviceToHost, s);
+        x.out = deep->out;
+        x.deep_len = deep->len;
+        x.deep_list = deep->list;
+        x.deep_count = deep->count;
     }
+    launch_scan_counts(s, T, tile_counts, tile_offsets, tile_stats, tile_temp, x);
     hipLaunchKernelGGL(packed ? k_emit_tiles<true> : k_emit_tiles<false>, dim3(8 + NS), dim3(kEmitThreads), 0, s,
                        tiles_x, tiles_y, sxn, super_offsets, k, r2, tile_offsets, ids,
                        std::max(1, num_isect / (4 * T)), tile_order);

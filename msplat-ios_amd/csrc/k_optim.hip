@@ -363,6 +363,21 @@ __global__ __launch_bounds__(256) void k_densify_copy_back(CopyArgs a) {
 
 inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
+__global__ void k_zero_counters(int *__restrict__ a, int na, int *__restrict__ b, int nb) {
+    for (int i = threadIdx.x; i < na; i += blockDim.x) a[i] = 0;
+    for (int i = threadIdx.x; i < nb; i += blockDim.x) b[i] = 0;
+}
+
+__global__ void k_step_report(const double *__restrict__ loss, const int *__restrict__ ctr, int n_ctr,
+                              mskern::Publish out) {
+    double *d = reinterpret_cast<double *>(out.data);
+    if (threadIdx.x < 2) d[threadIdx.x] = loss[threadIdx.x];
+    for (int i = threadIdx.x; i < n_ctr; i += blockDim.x) out.data[4 + i] = ctr[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(out.flag, out.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace
 
 namespace mskern {
@@ -384,6 +399,14 @@ void launch_zero16(hipStream_t s, float *p, int64_t n_float4) {
     if (n_float4 <= 0) return;
     const int64_t blocks = (n_float4 + 255) / 256;
     hipLaunchKernelGGL(k_zero16, dim3((unsigned)blocks), dim3(256), 0, s, reinterpret_cast<float4 *>(p), n_float4);
+}
+
+void launch_zero_counters(hipStream_t s, int *a, int na, int *b, int nb) {
+    hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(256), 0, s, a, na, b, nb);
+}
+
+void launch_step_report(hipStream_t s, const double *loss, const int *ctr, int n_ctr, const Publish &out) {
+    hipLaunchKernelGGL(k_step_report, dim3(1), dim3(256), 0, s, loss, ctr, n_ctr, out);
 }
 
 void launch_rgba8(hipStream_t s, const float *img, int64_t n, uint32_t *out) {

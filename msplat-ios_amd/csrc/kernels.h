@@ -49,6 +49,15 @@ void launch_project3d_bwd(hipStream_t s, const MsplatCamera &cam, const MsplatGa
 void launch_finish3d_grads(hipStream_t s, int n, const float *rec, float *g16);
 void launch_tiles_hit(hipStream_t s, const uint32_t *rect, const int *radii, int *out, int n);
 
+// Results that a kernel stores to pinned host memory while the stream goes
+// on; the host waits for *flag == seq (a system-scope release store after
+// `data`) instead of copying and draining the stream.
+struct Publish {
+    int *data = nullptr;  // pinned host memory; nullptr: nothing is published
+    int *flag = nullptr;
+    int seq = 0;
+};
+
 // k_binning.hip
 // Super-tiles are 4x4 tiles: sxn = ceil(tiles_x / 4), syn = ceil(tiles_y / 4),
 // NS = sxn * syn.  Scan temporaries: tile_scan_temp_ints(count) ints.
@@ -56,10 +65,12 @@ int64_t tile_scan_temp_ints(int T);
 // (splat, super-tile) pair counts -> super_counts[NS], super_offsets[NS + 1];
 // super_stats = {pairs, largest list, -, merge tiles of the huge lists},
 // zero on entry.
+// out.data receives {intersections (64-bit, *isect), pairs, largest list}.
 // super_cm (kBinMaxBlocks x NS ints) receives the per-(workgroup,
 // super-tile) key offsets that launch_bin_tiles places the keys at.
 void launch_super_count(hipStream_t s, int n, int tiles_x, int tiles_y, const int *radii, const uint32_t *rect,
-                        int *super_counts, int *super_offsets, int *super_cm, int *super_stats, int *temp);
+                        int *super_counts, int *super_offsets, int *super_cm, int *super_stats, int *temp,
+                        const unsigned long long *isect, const Publish &out);
 constexpr int kBinMaxBlocks = 256;
 // Scatter, per-super-tile sort, tile counts and offsets (tile_offsets[T + 1],
 // tile_stats = {intersections, largest tile}, zero on entry) and the
@@ -72,10 +83,11 @@ constexpr int kBinMaxBlocks = 256;
 // the order the rasterizers take the tiles in.
 // The deep-tile scan launch_bin_tiles queues once the tile offsets exist
 // (before the emission kernels): the tiles with at least `len` entries into
-// `list`, their number into *count, copied to *host_count.
+// `list`, their number into *count (zero on entry) and out.data[0].
 struct DeepScan {
     int len = 0;
-    int *list = nullptr, *count = nullptr, *host_count = nullptr;
+    int *list = nullptr, *count = nullptr;
+    Publish out;
 };
 void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int *radii, const uint32_t *rect,
                       const float *depths, const int *super_offsets, const int *super_cm, int super_max,
@@ -116,7 +128,7 @@ struct DeepTiles {
     float *tb = nullptr;
     int *cnt = nullptr;
     // the deep tiles run on `stream` between `fork` (recorded on the
-    // caller's stream) and `join` (waited on by the caller's stream); with
+    // caller's stream; `started` is where `stream` passes it) and `join` (waited on by the caller's stream); with
     // defer_log the forward's `join` follows the deep tiles' outputs only
     // and their blend logs (k_deep_log) are rebuilt after it on `stream`,
     // where the raster backward's deep part follows them (the caller's
@@ -126,7 +138,7 @@ struct DeepTiles {
     // of CUs by the per-tile launch (which would delay the deep part behind
     // the whole per-tile backward)
     hipStream_t stream = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr, logged = nullptr;
+    hipEvent_t fork = nullptr, started = nullptr, join = nullptr, logged = nullptr;
     bool defer_log = false;
 };
 void launch_deep_tiles(hipStream_t s, int T, const int *offsets, int deep_len, int *deep_list, int *count);
@@ -183,6 +195,11 @@ void launch_adam(hipStream_t s, float *p, const float *g, float *m, float *v, in
 void launch_clamp_max(hipStream_t s, float *p, int64_t n, float value);
 // p[0, 4 * n_float4) = 0; p 16-byte aligned.
 void launch_zero16(hipStream_t s, float *p, int64_t n_float4);
+// Zeroes two int arrays (a frame's counters) in one launch.
+void launch_zero_counters(hipStream_t s, int *a, int na, int *b, int nb);
+// Publishes the two loss doubles and the n_ctr counters (data: two doubles,
+// then the counters) behind everything queued on s.
+void launch_step_report(hipStream_t s, const double *loss, const int *ctr, int n_ctr, const Publish &out);
 int64_t scan_temp_ints(int64_t n);
 void launch_scan_i32(hipStream_t s, const int *in, int *out, int n, int *temp);
 
