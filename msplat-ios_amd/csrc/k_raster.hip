@@ -29,23 +29,27 @@ constexpr float kMScale = FAR_N / (FAR_N - NEAR_N);
 // MaskRec).  Planes: 0..2 the centred ray rows, centre and opacity
 // (eval_pair's p0..p2), 3 = (Tw, pos), 4 = (colour, gid), 5 = (normal, 0)
 // when NORMAL.
+struct SplatLoad {
+    float4 q0, q1, q2, q3, q4;
+    MaskRec m;
+};
+__device__ __forceinline__ SplatLoad fetch_splat(const float4 *__restrict__ rec, const float4 *__restrict__ mrec,
+                                                 int gid) {
+    const float4 *r = rec + 5 * (size_t)gid, *mr = mrec + 3 * (size_t)gid;
+    return {r[0], r[1], r[2], r[3], r[4], {mr[0], mr[1], mr[2]}};
+}
 template <bool NORMAL>
-__device__ __forceinline__ int load_batch(const float4 *__restrict__ rec, const float4 *__restrict__ mrec, int gid,
-                                          int pos, float4 *s_rec, float sx0, float sy0) {
-    const float4 *r = rec + 5 * (size_t)gid;
-    const float4 q0 = r[0], q1 = r[1], q2 = r[2], q3 = r[3], q4 = r[4];
-    const float4 *mr = mrec + 3 * (size_t)gid;
-    const MaskRec m = {mr[0], mr[1], mr[2]};
-    const f3 Tw = {q1.z, q1.w, q2.x};
+__device__ __forceinline__ int stage_splat(const SplatLoad &l, int gid, int pos, float4 *s_rec, float sx0, float sy0) {
+    const f3 Tw = {l.q1.z, l.q1.w, l.q2.x};
     f3 R0, nAx, nAy;
-    centred_rows({q0.x, q0.y, q0.z}, {q0.w, q1.x, q1.y}, Tw, q2.y, q2.z, R0, nAx, nAy);
+    centred_rows({l.q0.x, l.q0.y, l.q0.z}, {l.q0.w, l.q1.x, l.q1.y}, Tw, l.q2.y, l.q2.z, R0, nAx, nAy);
     s_rec[threadIdx.x] = make_float4(R0.x, R0.y, R0.z, nAx.x);
     s_rec[kThreads + threadIdx.x] = make_float4(nAx.y, nAx.z, nAy.x, nAy.y);
-    s_rec[2 * kThreads + threadIdx.x] = make_float4(nAy.z, q2.y, q2.z, q2.w);
+    s_rec[2 * kThreads + threadIdx.x] = make_float4(nAy.z, l.q2.y, l.q2.z, l.q2.w);
     s_rec[3 * kThreads + threadIdx.x] = make_float4(Tw.x, Tw.y, Tw.z, __int_as_float(pos));
-    s_rec[4 * kThreads + threadIdx.x] = make_float4(q3.w, q4.x, q4.y, __int_as_float(gid));
-    if (NORMAL) s_rec[5 * kThreads + threadIdx.x] = make_float4(q3.x, q3.y, q3.z, 0.f);
-    return quad_mask(m, q4.w, q2.y, q2.z, sx0, sy0);
+    s_rec[4 * kThreads + threadIdx.x] = make_float4(l.q3.w, l.q4.x, l.q4.y, __int_as_float(gid));
+    if (NORMAL) s_rec[5 * kThreads + threadIdx.x] = make_float4(l.q3.x, l.q3.y, l.q3.z, 0.f);
+    return quad_mask(l.m, l.q4.w, l.q2.y, l.q2.z, sx0, sy0);
 }
 
 // nd_rasterize_forward_2dgs_kernel (msplat_metal.metal:553-754).
@@ -65,13 +69,11 @@ __device__ __forceinline__ int load_batch(const float4 *__restrict__ rec, const 
 // indices, the depth, normal, alpha, median and distortion outputs and the
 // distortion moments are neither accumulated nor written.  Every
 // decision, and so every produced value, is the same as with FULL_OUT.
-// 7 waves per SIMD: the LDS of the image-only kernel allows 7 workgroups
-// per CU, and at most 72 VGPRs keep all of them resident (the compiler
-// would otherwise use more and fit 6; with two visits per iteration it
-// spills one value, reloaded once per batch, which costs less than the
-// seventh wave saves).
-template <bool LOG, bool FULL_OUT, bool COUNT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_raster_fwd(
+// V visits go through each step of the loop together: their evaluations do
+// not depend on each other, only their blends do.  AHEAD loads a batch's
+// splats while the batch before it is visited.
+template <bool LOG, bool FULL_OUT, bool COUNT, int V, bool AHEAD>
+__device__ __forceinline__ void raster_fwd(
     int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets,
     const int *__restrict__ ids, const float4 *__restrict__ rec, const float4 *__restrict__ mrec,
     const float *__restrict__ bgp, float *__restrict__ out_img, float *__restrict__ final_Ts, int *__restrict__ final_idx, float *__restrict__ out_depth,
@@ -120,79 +122,101 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(7, 8))
     __shared__ int s_vis[4];
     unsigned visits = 0, slots = 0;
     if (COUNT && threadIdx.x < 4) s_vis[threadIdx.x] = 0;
+    // AHEAD: the next batch's splats, and the ids of the one after it
+    const auto id_at = [&](int i) { return i < end ? ids[i] : 0; };
+    SplatLoad nl;
+    int gid_n = 0, gid_nn = 0;
+    if (AHEAD && end > start) {
+        gid_n = id_at(start + (int)threadIdx.x);
+        gid_nn = id_at(start + kThreads + (int)threadIdx.x);
+        nl = fetch_splat(rec, mrec, gid_n);
+    }
     for (int b0 = start; b0 < end; b0 += kThreads) {
         if (__syncthreads_and(done_m == ~0ull)) break;
         if (COUNT && threadIdx.x == 0)
             slots += 4u * (unsigned)max(max(s_vis[0], s_vis[1]), max(s_vis[2], s_vis[3]));
         const int idx = b0 + (int)threadIdx.x;
-        const int gid = idx < end ? ids[idx] : 0;
-        const int m = idx < end ? load_batch<FULL_OUT>(rec, mrec, gid, idx - start, s_rec, sx0, sy0) : 0;
+        int m = 0;
+        if (AHEAD) {
+            if (idx < end) m = stage_splat<FULL_OUT>(nl, gid_n, idx - start, s_rec, sx0, sy0);
+            gid_n = gid_nn;
+            if (b0 + kThreads < end) {
+                nl = fetch_splat(rec, mrec, gid_n);
+                gid_nn = id_at(idx + 2 * kThreads);
+            }
+        } else if (idx < end) {
+            const int gid = ids[idx];
+            m = stage_splat<FULL_OUT>(fetch_splat(rec, mrec, gid), gid, idx - start, s_rec, sx0, sy0);
+        }
         const int n = build_wave_lists(m, s_list, s_cnt);
         int nv = 0;
-        // one visit of slot list entry j; a visit after the wave is done
-        // changes nothing (no lane is active, so nothing blends or is logged)
-        const auto visit = [&](int j) {
-            if (COUNT) nv += done_m != ~0ull;
-            const int to = 16 * (int)s_list[wave][j];  // byte offset of the slot in a record plane
-            const auto plane = [&](int k) {
-                return *reinterpret_cast<const float4 *>(s_bytes + k * (kThreads * 16) + to);
-            };
-            // predicated: a lane that is done or rejects the pair adds
-            // colour * 0 (bit-identical sums) and keeps its state
-            if (COUNT) evals += __builtin_popcountll(~done_m);
-            const float4 q0 = plane(0), q1 = plane(1), q2 = plane(2), q3 = plane(3);
-            PairEval e;
-            const uint64_t act = eval_pair(px, py, q0, q1, q2, q3, e) & ~done_m;
-            const float next_T = Tr * (1.0f - e.alpha);
-            const uint64_t term = act & __builtin_amdgcn_ballot_w64(next_T <= 1e-4f);
-            const uint64_t bal = act & ~term;  // the lanes that blend the splat
-            done_m |= term;
-            const bool blend = __builtin_amdgcn_inverse_ballot_w64(bal);
-            const float w = blend ? e.alpha * Tr : 0.0f;
-            const float4 q4 = plane(4);
-            if (FULL_OUT) {
-                // 1-based list position of the splat (the reference's contributor count)
-                const int contrib = __float_as_int(q3.w) + 1;
-                const float A = 1.f - Tr;
-                const float dep_s = blend ? e.depth : 1.0f;  // finite stand-in off the blend
-                const float m_ = kMScale * (1.f - NEAR_N / dep_s);
-                dist = __builtin_fmaf(m_ * m_ * A + M2 - 2.f * m_ * M1, w, dist);
-                M1 = __builtin_fmaf(m_, w, M1);
-                M2 = __builtin_fmaf(m_ * m_, w, M2);
-                const bool med_now = blend & (Tr > 0.5f);
-                med = med_now ? e.depth : med;
-                med_c = med_now ? contrib : med_c;
-                dep = __builtin_fmaf(dep_s, w, dep);
-                const float4 q5 = plane(5);
-                nx = __builtin_fmaf(q5.x, w, nx);
-                ny = __builtin_fmaf(q5.y, w, ny);
-                nz = __builtin_fmaf(q5.z, w, nz);
-                last_c = blend ? contrib : last_c;
+        // a visit after the wave is done, or past the list's end (its last
+        // entry again), changes nothing: no lane is active, so nothing blends
+        // or is logged
+        for (int j = 0; j < n && done_m != ~0ull; j += V) {
+            float4 q0[V], q1[V], q2[V], q3[V], q4[V], q5[V];
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                const int to = 16 * (int)s_list[wave][min(j + u, n - 1)];  // byte offset of the slot in a record plane
+                const auto plane = [&](int k) {
+                    return *reinterpret_cast<const float4 *>(s_bytes + k * (kThreads * 16) + to);
+                };
+                q0[u] = plane(0), q1[u] = plane(1), q2[u] = plane(2), q3[u] = plane(3), q4[u] = plane(4);
+                if (FULL_OUT) q5[u] = plane(5);
             }
-            cr = __builtin_fmaf(q4.x, w, cr);
-            cg = __builtin_fmaf(q4.y, w, cg);
-            cb = __builtin_fmaf(q4.z, w, cb);
-            Tr = blend ? next_T : Tr;
-            if (COUNT) blends += __builtin_popcountll(bal);
-            if (LOG && bal) {
-                const bool mine = __builtin_amdgcn_inverse_ballot_w64(1ull << (nlog & 63));
-                lg_ent.x = mine ? (unsigned)bal : lg_ent.x;
-                lg_ent.y = mine ? (unsigned)(bal >> 32) : lg_ent.y;
-                lg_ent.z = mine ? __float_as_uint(q3.w) : lg_ent.z;
-                lg_ent.w = mine ? __float_as_uint(q4.w) : lg_ent.w;
-                // the transmittance before the next logged splat is the
-                // current one (a visit no lane blends changes nothing)
-                if ((++nlog & 63) == 0) lw.full(blog, lane, nlog, lg_ent, Tr);
+            PairEval ev[V];
+            uint64_t pass[V];
+            eval_pairs<V>(px, py, q0, q1, q2, q3, ev, pass);
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                const PairEval &e = ev[u];
+                const bool live = j + u < n;
+                if (COUNT) nv += live && done_m != ~0ull;
+                // predicated: a lane that is done or rejects the pair adds
+                // colour * 0 (bit-identical sums) and keeps its state
+                if (COUNT && live) evals += __builtin_popcountll(~done_m);
+                const uint64_t act = live ? pass[u] & ~done_m : 0ull;
+                const float next_T = Tr * (1.0f - e.alpha);
+                const uint64_t term = act & __builtin_amdgcn_ballot_w64(next_T <= 1e-4f);
+                const uint64_t bal = act & ~term;  // the lanes that blend the splat
+                done_m |= term;
+                const bool blend = __builtin_amdgcn_inverse_ballot_w64(bal);
+                const float w = blend ? e.alpha * Tr : 0.0f;
+                if (FULL_OUT) {
+                    // 1-based list position of the splat (the reference's contributor count)
+                    const int contrib = __float_as_int(q3[u].w) + 1;
+                    const float A = 1.f - Tr;
+                    const float dep_s = blend ? e.depth : 1.0f;  // finite stand-in off the blend
+                    const float m_ = kMScale * (1.f - NEAR_N / dep_s);
+                    dist = __builtin_fmaf(m_ * m_ * A + M2 - 2.f * m_ * M1, w, dist);
+                    M1 = __builtin_fmaf(m_, w, M1);
+                    M2 = __builtin_fmaf(m_ * m_, w, M2);
+                    const bool med_now = blend & (Tr > 0.5f);
+                    med = med_now ? e.depth : med;
+                    med_c = med_now ? contrib : med_c;
+                    dep = __builtin_fmaf(dep_s, w, dep);
+                    nx = __builtin_fmaf(q5[u].x, w, nx);
+                    ny = __builtin_fmaf(q5[u].y, w, ny);
+                    nz = __builtin_fmaf(q5[u].z, w, nz);
+                    last_c = blend ? contrib : last_c;
+                }
+                cr = __builtin_fmaf(q4[u].x, w, cr);
+                cg = __builtin_fmaf(q4[u].y, w, cg);
+                cb = __builtin_fmaf(q4[u].z, w, cb);
+                Tr = blend ? next_T : Tr;
+                if (COUNT) blends += __builtin_popcountll(bal);
+                if (LOG && bal) {
+                    const bool mine = __builtin_amdgcn_inverse_ballot_w64(1ull << (nlog & 63));
+                    lg_ent.x = mine ? (unsigned)bal : lg_ent.x;
+                    lg_ent.y = mine ? (unsigned)(bal >> 32) : lg_ent.y;
+                    lg_ent.z = mine ? __float_as_uint(q3[u].w) : lg_ent.z;
+                    lg_ent.w = mine ? __float_as_uint(q4[u].w) : lg_ent.w;
+                    // the transmittance before the next logged splat is the
+                    // current one (a visit no lane blends changes nothing)
+                    if ((++nlog & 63) == 0) lw.full(blog, lane, nlog, lg_ent, Tr);
+                }
             }
-        };
-        // two visits per iteration: the second's work up to alpha does not
-        // depend on the first's blend, so the two can be interleaved
-        int j = 0;
-        for (; j + 1 < n && done_m != ~0ull; j += 2) {
-            visit(j);
-            visit(j + 1);
         }
-        if (j < n && done_m != ~0ull) visit(j);
         if (COUNT) {
             visits += (unsigned)nv;
             if (lane == 0) s_vis[wave] = nv;
@@ -235,6 +259,36 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(7, 8))
     out_alpha[pix] = 1.f - Tr;
     out_median[pix] = med;
     out_dist[pix] = dist;
+}
+
+// 7 waves per SIMD: the LDS of the image-only kernel allows 7 workgroups
+// per CU, and at most 72 VGPRs keep all of them resident (the compiler
+// would otherwise use more and fit 6).
+template <bool LOG, bool FULL_OUT, bool COUNT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_raster_fwd(
+    int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets,
+    const int *__restrict__ ids, const float4 *__restrict__ rec, const float4 *__restrict__ mrec,
+    const float *__restrict__ bgp, float *__restrict__ out_img, float *__restrict__ final_Ts, int *__restrict__ final_idx, float *__restrict__ out_depth,
+    float *__restrict__ out_normal, float *__restrict__ out_alpha, float *__restrict__ out_median,
+    float *__restrict__ out_dist, unsigned long long *__restrict__ pair_counter, BlendLog blog, int deep_len) {
+    raster_fwd<LOG, FULL_OUT, COUNT, 2, false>(W, H, tiles_x, order, offsets, ids, rec, mrec, bgp, out_img, final_Ts, final_idx,
+                                         out_depth, out_normal, out_alpha, out_median, out_dist, pair_counter, blog,
+                                         deep_len);
+}
+
+// The same for frames of a few tiles per CU, whose waves have a SIMD to
+// themselves: four visits in flight and the next batch's loads hide what
+// other waves would.
+template <bool LOG, bool FULL_OUT, bool COUNT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 3))) void k_raster_fwd_few(
+    int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets,
+    const int *__restrict__ ids, const float4 *__restrict__ rec, const float4 *__restrict__ mrec,
+    const float *__restrict__ bgp, float *__restrict__ out_img, float *__restrict__ final_Ts, int *__restrict__ final_idx, float *__restrict__ out_depth,
+    float *__restrict__ out_normal, float *__restrict__ out_alpha, float *__restrict__ out_median,
+    float *__restrict__ out_dist, unsigned long long *__restrict__ pair_counter, BlendLog blog, int deep_len) {
+    raster_fwd<LOG, FULL_OUT, COUNT, 4, true>(W, H, tiles_x, order, offsets, ids, rec, mrec, bgp, out_img, final_Ts, final_idx,
+                                         out_depth, out_normal, out_alpha, out_median, out_dist, pair_counter, blog,
+                                         deep_len);
 }
 
 // nd_rasterize_backward_2dgs_kernel (msplat_metal.metal:1705-1979) over the
@@ -1001,6 +1055,9 @@ void launch_check_rcp(hipStream_t s, int efield, unsigned long long *bad) {
     hipLaunchKernelGGL(k_check_rcp, dim3((1u << 24) / 256), dim3(256), 0, s, (uint32_t)efield, bad);
 }
 
+// Frames whose tiles leave most of the chip's wave slots empty.  FEW_MEASURED
+static bool few_tiles(int tiles_x, int tiles_y) { return (int64_t)tiles_x * tiles_y <= 512; }
+
 void launch_raster_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets, const int *ids,
                        const float *rec, const float *mrec, const float *bg, float *out_img, float *final_Ts, int *final_idx,
                        float *out_depth, float *out_normal, float *out_alpha, float *out_median, float *out_dist,
@@ -1051,6 +1108,11 @@ void launch_raster_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, co
             full_outputs ? launch(k_raster_fwd<true, true, true>) : launch(k_raster_fwd<true, false, true>);
         else
             full_outputs ? launch(k_raster_fwd<false, true, true>) : launch(k_raster_fwd<false, false, true>);
+    } else if (few_tiles(tiles_x, tiles_y)) {
+        if (blog)
+            full_outputs ? launch(k_raster_fwd_few<true, true, false>) : launch(k_raster_fwd_few<true, false, false>);
+        else
+            full_outputs ? launch(k_raster_fwd_few<false, true, false>) : launch(k_raster_fwd_few<false, false, false>);
     } else {
         if (blog)
             full_outputs ? launch(k_raster_fwd<true, true, false>) : launch(k_raster_fwd<true, false, false>);

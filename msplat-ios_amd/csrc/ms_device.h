@@ -409,45 +409,71 @@ struct PairEval {
     float inv_z, u, v, rho3d, rho2d, depth, G, alpha;
 };
 
-__device__ __forceinline__ uint64_t eval_pair(float px, float py, const float4 &p0, const float4 &p1,
-                                              const float4 &p2, const float4 &p3, PairEval &e) {
+// V pairs of one pixel at once (V splats, the lane's pixel), so that their
+// chains overlap and share the reciprocal's range test.
+template <int V>
+__device__ __forceinline__ void eval_pairs(float px, float py, const float4 (&p0)[V], const float4 (&p1)[V],
+                                           const float4 (&p2)[V], const float4 (&p3)[V], PairEval (&e)[V],
+                                           uint64_t (&act)[V]) {
     // Straight-line: every value is computed, then the reference's
     // rejections are applied with their exact comparisons (a NaN compares
     // false in each, as in the reference's early returns), each as the
-    // wave's lane mask, so the wave needs no exec-mask branches.  Returns the
-    // mask of the wave's lanes whose pair passes; called by the whole wave.
-    const float dxs = p2.y - px, dys = p2.z - py;
-    e.ray = {__builtin_fmaf(dxs, p0.w, __builtin_fmaf(dys, p1.z, p0.x)),
-             __builtin_fmaf(dxs, p1.x, __builtin_fmaf(dys, p1.w, p0.y)),
-             __builtin_fmaf(dxs, p1.y, __builtin_fmaf(dys, p2.x, p0.z))};
-    // infinite when ray.z == 0; that pair is rejected below
-    e.inv_z = ms_rcp_nr(e.ray.z);
-    {
-        // the division only where some lane's ray.z is outside the exact
-        // range (a wave-uniform branch, so the common case skips it)
-        const bool odd = !ms_rcp_nr_exact(e.ray.z);
-        if (__builtin_amdgcn_ballot_w64(odd)) {
-            float z = e.ray.z;
+    // wave's lane mask, so the wave needs no exec-mask branches.  act[u] is
+    // the mask of the wave's lanes whose pair passes; called by the whole
+    // wave.
+    float dxs[V], dys[V];
+    bool odd = false;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        dxs[u] = p2[u].y - px;
+        dys[u] = p2[u].z - py;
+        e[u].ray = {__builtin_fmaf(dxs[u], p0[u].w, __builtin_fmaf(dys[u], p1[u].z, p0[u].x)),
+                    __builtin_fmaf(dxs[u], p1[u].x, __builtin_fmaf(dys[u], p1[u].w, p0[u].y)),
+                    __builtin_fmaf(dxs[u], p1[u].y, __builtin_fmaf(dys[u], p2[u].x, p0[u].z))};
+        // infinite when ray.z == 0; that pair is rejected below
+        e[u].inv_z = ms_rcp_nr(e[u].ray.z);
+        odd |= !ms_rcp_nr_exact(e[u].ray.z);
+    }
+    // the division only where some lane's ray.z is outside the exact range
+    // (a wave-uniform branch, so the common case skips it)
+    if (__builtin_amdgcn_ballot_w64(odd)) {
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            float z = e[u].ray.z;
             asm volatile("" : "+v"(z));  // keeps the division inside the branch
-            if (odd) e.inv_z = 1.0f / z;
+            if (!ms_rcp_nr_exact(z)) e[u].inv_z = 1.0f / z;
         }
     }
-    e.u = e.ray.x * e.inv_z;
-    e.v = e.ray.y * e.inv_z;
-    e.rho3d = __builtin_fmaf(e.u, e.u, e.v * e.v);
-    e.rho2d = FILTER_INV_SQ * __builtin_fmaf(dxs, dxs, dys * dys);
-    // capped for ms_gauss_capped (one v_min3): beyond the cap ms_gauss is
-    // below 1e-37, so alpha < 1/255 either way and every decision, hence
-    // every output, is the one ms_gauss(min(rho3d, rho2d)) gives
-    const float rho = __builtin_fminf(__builtin_fminf(e.rho3d, e.rho2d), kGaussRhoCap);
-    e.depth = __builtin_fmaf(e.u, p3.x, __builtin_fmaf(e.v, p3.y, p3.z));
-    // The reference's power > 0 rejection (msplat_metal.metal:676-677) never
-    // fires: rho is a minimum of sums of squares (>= 0, +inf or NaN), so
-    // power = -rho / 2 is <= 0, -inf or NaN.
-    e.G = ms_gauss_capped(rho);
-    e.alpha = __builtin_fminf(0.99f, p2.w * e.G);
-    return __builtin_amdgcn_ballot_w64(!(e.ray.z == 0.0f)) & __builtin_amdgcn_ballot_w64(!(e.depth < NEAR_N)) &
-           __builtin_amdgcn_ballot_w64(!(e.alpha < 1.0f / 255.0f));
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        e[u].u = e[u].ray.x * e[u].inv_z;
+        e[u].v = e[u].ray.y * e[u].inv_z;
+        e[u].rho3d = __builtin_fmaf(e[u].u, e[u].u, e[u].v * e[u].v);
+        e[u].rho2d = FILTER_INV_SQ * __builtin_fmaf(dxs[u], dxs[u], dys[u] * dys[u]);
+        // capped for ms_gauss_capped (one v_min3): beyond the cap ms_gauss is
+        // below 1e-37, so alpha < 1/255 either way and every decision, hence
+        // every output, is the one ms_gauss(min(rho3d, rho2d)) gives
+        const float rho = __builtin_fminf(__builtin_fminf(e[u].rho3d, e[u].rho2d), kGaussRhoCap);
+        e[u].depth = __builtin_fmaf(e[u].u, p3[u].x, __builtin_fmaf(e[u].v, p3[u].y, p3[u].z));
+        // The reference's power > 0 rejection (msplat_metal.metal:676-677)
+        // never fires: rho is a minimum of sums of squares (>= 0, +inf or
+        // NaN), so power = -rho / 2 is <= 0, -inf or NaN.
+        e[u].G = ms_gauss_capped(rho);
+        e[u].alpha = __builtin_fminf(0.99f, p2[u].w * e[u].G);
+        act[u] = __builtin_amdgcn_ballot_w64(!(e[u].ray.z == 0.0f)) &
+                 __builtin_amdgcn_ballot_w64(!(e[u].depth < NEAR_N)) &
+                 __builtin_amdgcn_ballot_w64(!(e[u].alpha < 1.0f / 255.0f));
+    }
+}
+
+__device__ __forceinline__ uint64_t eval_pair(float px, float py, const float4 &p0, const float4 &p1,
+                                              const float4 &p2, const float4 &p3, PairEval &e) {
+    const float4 a0[1] = {p0}, a1[1] = {p1}, a2[1] = {p2}, a3[1] = {p3};
+    PairEval ev[1];
+    uint64_t act[1];
+    eval_pairs<1>(px, py, a0, a1, a2, a3, ev, act);
+    e = ev[0];
+    return act[0];
 }
 
 // Pixels of a 16x16 tile handled by wave w of a 256-thread rasterizer
