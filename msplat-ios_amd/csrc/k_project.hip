@@ -296,7 +296,9 @@ __device__ __forceinline__ void moments_to_dT(f3 Tu, f3 Tv, f3 Tw, float xs, flo
 // (1 - opacity) (msplat_metal.metal:1976), the colour sums masked where the
 // colour was clamped at zero (:1873-1880; the record holds the clamped
 // colour, positive exactly where the clamp passes the gradient).  Then the
-// moments become dL/dtransMat.
+// moments become dL/dtransMat, and the sums of dL/ddepth (u, v, 1) that a
+// distortion term leaves in the normal's slots (zero otherwise) join the
+// gradient of the depth row Tw.
 __device__ __forceinline__ void finish_image_grads(f3 Tu, f3 Tv, f3 Tw, float4 q2, float4 q3, float4 q4,
                                                    float g[16]) {
     const float opa = q2.w;
@@ -307,6 +309,11 @@ __device__ __forceinline__ void finish_image_grads(f3 Tu, f3 Tv, f3 Tw, float4 q
     g[14] = q4.x > 0.0f ? g[14] : 0.0f;
     g[15] = q4.y > 0.0f ? g[15] : 0.0f;
     moments_to_dT(Tu, Tv, Tw, q2.y, q2.z, g);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        g[6 + k] += g[9 + k];
+        g[9 + k] = 0.f;
+    }
 }
 
 // project_and_sh_backward_2dgs_kernel (msplat_metal.metal:2003-2209).

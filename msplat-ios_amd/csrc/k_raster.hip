@@ -309,35 +309,295 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 3))
 // The 16 per-splat gradients [dL_dtransMat 9, dL_dnormal3D 3, dL_dopacity,
 // dL_dcolors 3] are reduced across the wave and added with one 16-lane
 // global float atomic (one 64-byte line) per (wave, splat).
-// FULL = false is the training step's case: the only upstream gradient is
-// dL/dimage, so the depth / alpha / normal / median / distortion terms are
-// compiled out and the colour suffix is carried as its projection on
-// dL/dimage.  Its grads16 rows hold per-splat sums without their per-splat
-// factors: the nine ray moments without -opacity, the opacity-logit sum
-// without opacity (1 - opacity), the colour sums without the clamp mask;
+// k_raster_bwd_full takes any upstream gradients.  The training step's case,
+// where they are dL/dimage and (DIST) a uniform dL/ddistortion, has its own
+// kernels (raster_bwd), without the depth / alpha / normal / median terms and
+// with the colour suffix carried as its projection on dL/dimage.  Their
+// grads16 rows hold per-splat sums without their per-splat factors: the nine
+// ray moments without -opacity, the opacity-logit sum without opacity (1 -
+// opacity), the colour sums without the clamp mask, and in slots 9..11 (the
+// normal's, otherwise zero) the sums of dL/ddepth times (u, v, 1);
 // finish_image_grads applies them once per splat.
-template <bool FULL>
-struct BwdLds;
-template <>
-struct BwdLds<true> {
-    float4 r[4][7][64];
-    uint4 e[4][64];
-};
-template <>
-struct BwdLds<false> {
-    float4 r[4][4][32];
-    float red[4][512];
+//
+// V log entries go through each step of the loop together: their evaluations
+// do not depend on each other, only the transmittance and the suffix do.
+
+// The reduction's slots: 13 non-zero sums in five permlane pairs (rows 0, 2,
+// 4, 6, 7) and three raw rows (1, 3, 5), so five permlane swaps per visit
+// instead of seven; with DIST 16 sums in eight pairs.  Nibble k of the grads16
+// index of reduction slot k (the unused upper slots of raw rows read 0).
+template <bool DIST>
+struct BwdSlots {
+    static constexpr unsigned kRaw = DIST ? 0u : 0x2Au;
+    static constexpr unsigned long long kGrad = DIST ? 0xfebca398d7654210ull : 0xfe0c0308d7654210ull;
 };
 
-// The image-only reduction's slots: 13 non-zero sums in five permlane pairs
-// (rows 0, 2, 4, 6, 7) and three raw rows (1, 3, 5), so five permlane swaps
-// per visit instead of seven.  Nibble k of kImgGrad is the grads16 index of
-// reduction slot k (the unused upper slots of raw rows read 0).
-constexpr unsigned kImgRaw = 0x2A;
-constexpr unsigned long long kImgGrad = 0xfe0c0308d7654210ull;
+template <bool DIST, int V, bool AHEAD>
+__device__ __forceinline__ void raster_bwd(
+    int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets, const BlendLog &blog,
+    const float4 *__restrict__ rec, const float *__restrict__ bgp, const float *__restrict__ final_Ts,
+    const float *__restrict__ dL_dimg, float dreg, float *__restrict__ grads16, int deep_len) {
+    // order: every tile, or the deep tiles (their own launch)
+    const int tile = order[blockIdx.x];
+    if (tile < 0) return;
+    const int start = offsets[tile], len = offsets[tile + 1] - start;
+    if (len >= deep_len) return;
+    if (overflowed(blog)) return;  // an incomplete log: the step is redone with a larger pool
+    // entries staged per chunk: 32, so that with V = 1 (16 KB of LDS per
+    // workgroup) the registers, not LDS, set the waves per SIMD
+    constexpr int kWave = 64, kChunk = 32, kPlanes = DIST ? 5 : 4;
+    constexpr unsigned kRaw = BwdSlots<DIST>::kRaw;
+    __shared__ float4 s_r[4][kPlanes][kChunk];
+    __shared__ float s_red[4][V][512];
+    const int lane = threadIdx.x & 63;
+    // uniform, so that the log entries are scalar loads
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tx = tile % tiles_x, ty = tile / tiles_x;
+    const int pxi = tx * 16 + lane_px(wave, lane);
+    const int pyi = ty * 16 + lane_py(wave, lane);
+    const bool inside = pxi < W && pyi < H;
+    const float px = (float)pxi, py = (float)pyi;
+    const int nlog = __builtin_amdgcn_readfirstlane(blog.wave_cnt[4 * tile + wave]);
+    Red8<kRaw> red8;
+    red8.init(&s_red[wave][0][0], lane);
+    const int *__restrict__ chunk_of = blog.table + log_table_base(start, len, tile, wave);
+    const size_t pix = inside ? (size_t)pyi * W + pxi : 0;
+    float T_final = 1.f, dp0 = 0.f, dp1 = 0.f, dp2 = 0.f, fD = 0.f, fD2 = 0.f;
+    if (inside) {
+        T_final = final_Ts[3 * pix];
+        dp0 = dL_dimg[3 * pix];
+        dp1 = dL_dimg[3 * pix + 1];
+        dp2 = dL_dimg[3 * pix + 2];
+        if (DIST) {
+            fD = final_Ts[3 * pix + 1];
+            fD2 = final_Ts[3 * pix + 2];
+        }
+    }
+    const float fA = 1.0f - T_final;
+    const float bgT = -T_final * (bgp[0] * dp0 + bgp[1] * dp1 + bgp[2] * dp2);
+    // only the lanes red8.adds marks hold a whole sum
+    const int gi = (int)((BwdSlots<DIST>::kGrad >> (4 * red8.slot)) & 15u);
 
-template <bool FULL>
+    float acc_v = 0.f;  // the suffix of the reference's recurrences, updated as soon as a splat is done
+    const int nchunks = (nlog + kChunk - 1) / kChunk;
+    float Tr = T_final;
+    // A chunk's loads depend on each other (pool chunk id, log entry, splat
+    // record), so they are issued ahead: the pool chunk ids 64 at a time (lane
+    // l holds id 64 cgrp + l), the splat ids one chunk ahead (two with AHEAD),
+    // the checkpoint one chunk ahead, and with AHEAD the records too.
+    const int npool = (nlog + kWave - 1) / kWave;
+    int cgrp = max(npool - 1, 0) >> 6;
+    const auto load_ids = [&] { return 64 * cgrp + lane < npool ? chunk_of[64 * cgrp + lane] : 0; };
+    int cids = load_ids();
+    const auto pool_chunk = [&](int c) {  // of chunk c, asked for in descending order
+        const int k = max(c, 0) * kChunk / kWave;
+        if ((k >> 6) != cgrp) {
+            cgrp = k >> 6;
+            cids = load_ids();
+        }
+        return __builtin_amdgcn_readlane(cids, k & 63);
+    };
+    const auto entries = [&](int c, int cid) { return blog.ent + 64 * (size_t)cid + (max(c, 0) * kChunk & (kWave - 1)); };
+    const auto gid_at = [&](int c, const uint4 *e) { return max(c, 0) * kChunk + lane < nlog && lane < kChunk ? (int)e[lane].w : 0; };
+    struct Rec {
+        float4 q0, q1, q2, q3, q4;
+    };
+    const auto fetch = [&](int gid) {
+        const float4 *r = rec + 5 * (size_t)gid;
+        return Rec{r[0], r[1], r[2], r[3], r[4]};
+    };
+    int cid_n = 0, gid_n = 0, gid_nn = 0;
+    const uint4 *lg_n = blog.ent, *lg_nn = blog.ent;
+    float ck_n = 0.f;
+    Rec rec_n;
+    if (nchunks > 0) {
+        cid_n = pool_chunk(nchunks - 1);
+        lg_n = entries(nchunks - 1, cid_n);
+        gid_n = gid_at(nchunks - 1, lg_n);
+        if (AHEAD) {
+            const int cid = pool_chunk(nchunks - 2);
+            lg_nn = entries(nchunks - 2, cid);
+            gid_nn = gid_at(nchunks - 2, lg_nn);
+            rec_n = fetch(gid_n);
+            cid_n = cid;
+        }
+    }
+    for (int c = nchunks - 1; c >= 0; --c) {
+        const int c0 = c * kChunk;
+        const int m = min(kChunk, nlog - c0);
+        // the pool chunk holding entries c0 .. c0 + m - 1, and its checkpoint:
+        // the transmittance after the chunk's last splat is the final
+        // transmittance, the prefix checkpoint of the entry after it when
+        // that entry is a multiple of 64, else the value the recurrence of
+        // the chunk after it ended with (the same operations in the same
+        // order as one 64-entry chunk)
+        const uint4 *__restrict__ lg = lg_n;
+        if (c != nchunks - 1 && ((c0 + kChunk) & (kWave - 1)) == 0) Tr = ck_n;
+        const Rec r = AHEAD ? rec_n : fetch(gid_n);
+        if (AHEAD) {
+            lg_n = lg_nn;
+            gid_n = gid_nn;
+            // chunk c - 1 ends its pool chunk (whose id cid_n is)
+            if ((c0 & (kWave - 1)) == 0 && c > 0) ck_n = blog.ckpt[64 * (size_t)cid_n + lane];
+            if (c > 0) rec_n = fetch(gid_n);
+            cid_n = pool_chunk(c - 2);
+            lg_nn = entries(c - 2, cid_n);
+            gid_nn = gid_at(c - 2, lg_nn);
+        } else if (c > 0) {
+            cid_n = pool_chunk(c - 1);
+            if ((c0 & (kWave - 1)) == 0) ck_n = blog.ckpt[64 * (size_t)cid_n + lane];
+            lg_n = entries(c - 1, cid_n);
+            gid_n = gid_at(c - 1, lg_n);
+        }
+        if (lane < m) {
+            // the forward's centred ray rows (centred_rows), then the colour
+            const float4 q0 = r.q0, q1 = r.q1, q2 = r.q2, q3 = r.q3, q4 = r.q4;
+            f3 R0, nAx, nAy;
+            centred_rows({q0.x, q0.y, q0.z}, {q0.w, q1.x, q1.y}, {q1.z, q1.w, q2.x}, q2.y, q2.z, R0, nAx, nAy);
+            s_r[wave][0][lane] = make_float4(R0.x, R0.y, R0.z, nAx.x);
+            s_r[wave][1][lane] = make_float4(nAx.y, nAx.z, nAy.x, nAy.y);
+            s_r[wave][2][lane] = make_float4(nAy.z, q2.y, q2.z, q2.w);
+            s_r[wave][3][lane] = make_float4(q3.w, q4.x, q4.y, 0.f);
+            // a logged splat blended somewhere, so its opacity is at least 1/255
+            if constexpr (DIST) s_r[wave][4][lane] = make_float4(q1.z, q1.w, q2.x, 1.0f / q2.w);
+        }
+        wave_lds_sync();
+        // the entries' addresses are uniform (scalar loads), each group
+        // fetched one step ahead so its latency is not waited on, and an
+        // entry's ballot is the lane mask of `has` itself
+        uint4 e_next[V];
+#pragma unroll
+        for (int u = 0; u < V; ++u) e_next[u] = lg[max(m - 1 - u, 0)];
+        for (int j = m - 1; j >= 0; j -= V) {
+            uint4 en[V];
+            float dxs[V], dys[V], inv_z[V], uu[V], vv[V], G[V], alpha[V], inv_om[V], depth[V];
+            float4 col[V], tw[V];
+            bool has[V], use3d[V];
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                en[u] = e_next[u];
+                e_next[u] = lg[max(j - V - u, 0)];
+            }
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                const int q = max(j - u, 0);
+                has[u] = __builtin_amdgcn_inverse_ballot_w64(j - u >= 0 ? ((uint64_t)en[u].y << 32) | en[u].x : 0ull);
+                const float4 q0 = s_r[wave][0][q], q1 = s_r[wave][1][q], q2 = s_r[wave][2][q];
+                col[u] = s_r[wave][3][q];
+                if constexpr (DIST) tw[u] = s_r[wave][4][q];
+                const float opa = q2.w;
+                dxs[u] = q2.y - px;
+                dys[u] = q2.z - py;
+                const float rx = __builtin_fmaf(dxs[u], q0.w, __builtin_fmaf(dys[u], q1.z, q0.x));
+                const float ry = __builtin_fmaf(dxs[u], q1.x, __builtin_fmaf(dys[u], q1.w, q0.y));
+                const float rz = __builtin_fmaf(dxs[u], q1.y, __builtin_fmaf(dys[u], q2.x, q0.z));
+                inv_z[u] = has[u] ? __builtin_amdgcn_rcpf(rz) : 0.f;
+                uu[u] = rx * inv_z[u];
+                vv[u] = ry * inv_z[u];
+                const float rho3d = __builtin_fmaf(uu[u], uu[u], vv[u] * vv[u]);
+                const float rho2d = FILTER_INV_SQ * __builtin_fmaf(dxs[u], dxs[u], dys[u] * dys[u]);
+                use3d[u] = rho3d <= rho2d;
+                // zero where the lane did not blend: alpha, the transmittance
+                // factor, the suffix update and every gradient term follow
+                G[u] = has[u] ? __builtin_amdgcn_exp2f(__builtin_fminf(rho3d, rho2d) * -0.72134752044448170368f) : 0.f;
+                alpha[u] = __builtin_fminf(0.99f, opa * G[u]);
+                inv_om[u] = __builtin_amdgcn_rcpf(1.0f - alpha[u]);
+                // lanes that did not blend get a finite stand-in
+                if constexpr (DIST)
+                    depth[u] = has[u] ? __builtin_fmaf(uu[u], tw[u].x, __builtin_fmaf(vv[u], tw[u].y, tw[u].z)) : 1.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                Tr *= inv_om[u];  // transmittance before this splat (unchanged where it did not blend)
+                const float aT = alpha[u] * Tr;
+                // dL/dimage . colour
+                float vl = __builtin_fmaf(dp0, col[u].x, __builtin_fmaf(dp1, col[u].y, dp2 * col[u].z));
+                float dz = 0.f;
+                if constexpr (DIST) {
+                    // the distortion's dL/dweight has the colours' recurrence
+                    // (:1887-1894), so it joins their projection
+                    const float inv_d = __builtin_amdgcn_rcpf(depth[u]);
+                    const float m_d = kMScale * (1.0f - NEAR_N * inv_d);
+                    const float dmd_dd = (FAR_N * NEAR_N) / (FAR_N - NEAR_N) * inv_d * inv_d;
+                    vl += (fD2 + m_d * m_d * fA - 2.0f * m_d * fD) * dreg;
+                    dz = 2.0f * aT * (m_d * fA - fD) * dreg * dmd_dd;
+                }
+                // acc_v is the suffix behind this splat.  The reference
+                // folds a splat in when the next blended splat is reached
+                // (last_alpha / last_color, :1875-1876, :1919); folding it
+                // in as soon as it is done uses the same values, and
+                // alpha = 0 leaves the suffix unchanged without a select
+                const float dv = vl - acc_v;
+                const float dLda = __builtin_fmaf(dv, Tr, bgT * inv_om[u]);
+                acc_v = __builtin_fmaf(alpha[u], dv, acc_v);
+                const float gg = dLda * G[u];
+                // dL/d(ray), up to the factor -opa, on the 3D branch: the
+                // ray-splat point's gradient (gg u, gg v), and with DIST -dz
+                // / opa of the depth's, / ray.z pulled back through (u, v) =
+                // ray.xy / ray.z; its moments over the wave's pixels
+                // about the splat centre (sum dp, sum (xs - px) dp,
+                // sum (ys - py) dp) determine the nine transMat gradients
+                float dsx, dsy;
+                if constexpr (DIST) {
+                    const float zo = dz * tw[u].w;
+                    dsx = use3d[u] ? __builtin_fmaf(gg, uu[u], -zo * tw[u].x) * inv_z[u] : 0.f;
+                    dsy = use3d[u] ? __builtin_fmaf(gg, vv[u], -zo * tw[u].y) * inv_z[u] : 0.f;
+                } else {
+                    const float t = (use3d[u] ? gg : 0.f) * inv_z[u];
+                    dsx = t * uu[u];
+                    dsy = t * vv[u];
+                }
+                const float dpz = use3d[u] || !DIST ? -__builtin_fmaf(dsx, uu[u], dsy * vv[u]) : 0.f;
+                float v16[16];
+                // reduction slots (BwdSlots): pairs (0, 8), (2, 10), (4, 12),
+                // (6, 14), (7, 15) and rows 1, 3, 5
+                v16[0] = dsx;
+                v16[8] = dys[u] * dpz;
+                v16[1] = dsy;
+                v16[2] = dpz;
+                v16[10] = dxs[u] * dsx;
+                v16[3] = dxs[u] * dsy;
+                v16[4] = dxs[u] * dpz;
+                v16[12] = gg;
+                v16[5] = dys[u] * dsx;
+                v16[6] = dys[u] * dsy;
+                v16[14] = aT * dp1;
+                v16[7] = aT * dp0;
+                v16[15] = aT * dp2;
+                v16[9] = DIST ? uu[u] * dz : 0.f;
+                v16[11] = DIST ? vv[u] * dz : 0.f;
+                v16[13] = dz;
+                reduce16_write(v16, red8, 512 * u);
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                const float s = reduce16_read(red8, 512 * u);
+                if (j - u >= 0 && red8.adds && s != 0.f) unsafeAtomicAdd(&grads16[(size_t)en[u].w * 16 + gi], s);
+            }
+            wave_lds_sync();
+        }
+    }
+}
+
+template <bool DIST>
 __global__ __launch_bounds__(kThreads) void k_raster_bwd(
+    int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets, BlendLog blog,
+    const float4 *__restrict__ rec, const float *__restrict__ bgp, const float *__restrict__ final_Ts,
+    const float *__restrict__ dL_dimg, float dreg, float *__restrict__ grads16, int deep_len) {
+    raster_bwd<DIST, 1, false>(W, H, tiles_x, order, offsets, blog, rec, bgp, final_Ts, dL_dimg, dreg, grads16, deep_len);
+}
+
+// Frames of a few tiles per CU (few_tiles): two entries in flight.
+template <bool DIST>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 3))) void k_raster_bwd_few(
+    int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets, BlendLog blog,
+    const float4 *__restrict__ rec, const float *__restrict__ bgp, const float *__restrict__ final_Ts,
+    const float *__restrict__ dL_dimg, float dreg, float *__restrict__ grads16, int deep_len) {
+    raster_bwd<DIST, 2, true>(W, H, tiles_x, order, offsets, blog, rec, bgp, final_Ts, dL_dimg, dreg, grads16, deep_len);
+}
+
+__global__ __launch_bounds__(kThreads) void k_raster_bwd_full(
     int W, int H, int tiles_x, const int *__restrict__ order, const int *__restrict__ offsets, BlendLog blog, const float4 *__restrict__ rec,
     const float *__restrict__ bgp, const float *__restrict__ final_Ts, const int *__restrict__ final_idx,
     const float *__restrict__ dL_dimg, const float *__restrict__ dL_ddepth, const float *__restrict__ dL_daccum,
@@ -349,14 +609,10 @@ __global__ __launch_bounds__(kThreads) void k_raster_bwd(
     if (offsets[tile + 1] - offsets[tile] >= deep_len) return;
     if (overflowed(blog)) return;  // an incomplete log: the step is redone with a larger pool
     constexpr int kWave = 64;
-    // per wave: the staged entries' record planes (the image-only path
-    // stages 4, the full one 7) and the log entries (full) or the reduction
-    // scratch (image-only, wave_reduce16_lds8); 16 KB per workgroup for the
-    // image-only kernel
-    __shared__ BwdLds<FULL> L;
-    auto &s_r = L.r;
+    // per wave: the staged entries' record planes and the log entries
+    __shared__ float4 s_r[4][7][64];
+    __shared__ uint4 s_e[4][64];
     const int lane = threadIdx.x & 63;
-    // uniform, so that the log entries of the image-only loop are scalar loads
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tx = tile % tiles_x, ty = tile / tiles_x;
     const int pxi = tx * 16 + lane_px(wave, lane);
@@ -365,8 +621,6 @@ __global__ __launch_bounds__(kThreads) void k_raster_bwd(
     const float px = (float)pxi, py = (float)pyi;
     const int start = offsets[tile], len = offsets[tile + 1] - start;
     const int nlog = __builtin_amdgcn_readfirstlane(blog.wave_cnt[4 * tile + wave]);
-    Red8<kImgRaw> red8;
-    if (!FULL) red8.init(reinterpret_cast<float *>(&L) + sizeof(L.r) / sizeof(float) + wave * 512, lane);
     const int *__restrict__ chunk_of = blog.table + log_table_base(start, len, tile, wave);
     const size_t pix = inside ? (size_t)pyi * W + pxi : 0;
 
@@ -379,150 +633,64 @@ __global__ __launch_bounds__(kThreads) void k_raster_bwd(
         dp0 = dL_dimg[3 * pix];
         dp1 = dL_dimg[3 * pix + 1];
         dp2 = dL_dimg[3 * pix + 2];
-        if (FULL) {
-            fD = final_Ts[3 * pix + 1];
-            fD2 = final_Ts[3 * pix + 2];
-            med_pos = final_idx[2 * pix + 1] - 1;
-            if (dL_ddepth) ddep = dL_ddepth[pix];
-            if (dL_daccum) dacc = dL_daccum[pix];
-            if (dL_dnormal) {
-                dn0 = dL_dnormal[3 * pix];
-                dn1 = dL_dnormal[3 * pix + 1];
-                dn2 = dL_dnormal[3 * pix + 2];
-            }
-            if (dL_dmedian) dmed = dL_dmedian[pix];
-            dreg = dL_ddist ? dL_ddist[pix] : ddist_uniform;
+        fD = final_Ts[3 * pix + 1];
+        fD2 = final_Ts[3 * pix + 2];
+        med_pos = final_idx[2 * pix + 1] - 1;
+        if (dL_ddepth) ddep = dL_ddepth[pix];
+        if (dL_daccum) dacc = dL_daccum[pix];
+        if (dL_dnormal) {
+            dn0 = dL_dnormal[3 * pix];
+            dn1 = dL_dnormal[3 * pix + 1];
+            dn2 = dL_dnormal[3 * pix + 2];
         }
+        if (dL_dmedian) dmed = dL_dmedian[pix];
+        dreg = dL_ddist ? dL_ddist[pix] : ddist_uniform;
     }
     const float fA = 1.0f - T_final;
     const float bgT = -T_final * (bgp[0] * dp0 + bgp[1] * dp1 + bgp[2] * dp2);
-    // lane l of the reduction ends with slot vi (see wave_reduce16), which
-    // holds grads16 index gi (image-only: slot red8.slot, its index in
-    // kImgGrad; only the lanes red8.adds marks hold a whole sum)
-    const int vi = ((lane >> 5) & 1) * 8 + ((lane >> 4) & 1) * 4 + ((lane >> 3) & 1) * 2 + ((lane >> 2) & 1);
-    const int gi = FULL ? vi : (int)((kImgGrad >> (4 * red8.slot)) & 15u);
-    const bool adds = FULL ? (lane & 3) == 0 : red8.adds;
+    // lane l of the reduction ends with grads16 index gi (see wave_reduce16)
+    const int gi = ((lane >> 5) & 1) * 8 + ((lane >> 4) & 1) * 4 + ((lane >> 3) & 1) * 2 + ((lane >> 2) & 1);
 
-    // suffix state of the reference's recurrences (image-only: the colour
-    // suffix projected on dL/dimage, updated as soon as a splat is done)
-    float last_alpha = 0.f, acc_v = 0.f;
+    // suffix state of the reference's recurrences
+    float last_alpha = 0.f;
     float acc_c[3] = {0.f, 0.f, 0.f}, last_c[3] = {0.f, 0.f, 0.f};
     float acc_d = 0.f, last_d = 0.f, acc_a = 0.f, last_dLdT = 0.f;
     float acc_n[3] = {0.f, 0.f, 0.f}, last_n[3] = {0.f, 0.f, 0.f};
 
-    // entries staged per chunk: 64 (full), 32 (image-only: 16 KB of LDS per
-    // workgroup, so that its 52 VGPRs, not LDS, set the waves per SIMD)
-    constexpr int kChunk = FULL ? kWave : kWave / 2;
+    constexpr int kChunk = kWave;  // entries staged per chunk
     const int nchunks = (nlog + kChunk - 1) / kChunk;
     float Tr = T_final;
     for (int c = nchunks - 1; c >= 0; --c) {
         const int c0 = c * kChunk;
         const int m = min(kChunk, nlog - c0);
-        // transmittance after the chunk's last splat: the final
-        // transmittance, the prefix checkpoint of the entry after it when
-        // that entry is a multiple of 64, else the value the recurrence of
-        // the chunk after it ended with (the same operations in the same
-        // order as one 64-entry chunk)
         // the pool chunk holding entries c0 .. c0 + m - 1, and its checkpoint
+        // (the transmittance before the entry after them)
         const int cid = __builtin_amdgcn_readfirstlane(chunk_of[c0 >> 6]);
-        const uint4 *__restrict__ lg = blog.ent + 64 * (size_t)cid + (c0 & 63);
-        if (c != nchunks - 1 && ((c0 + kChunk) & (kWave - 1)) == 0) Tr = blog.ckpt[64 * (size_t)cid + lane];
+        const uint4 *__restrict__ lg = blog.ent + 64 * (size_t)cid;
+        if (c != nchunks - 1) Tr = blog.ckpt[64 * (size_t)cid + lane];
         if (lane < m) {
             const uint4 e = lg[lane];
             const float4 *r = rec + 5 * (size_t)e.w;
-            // the forward's centred ray rows (centred_rows), then the colour;
-            // the full case adds the raw transMat rows and the normal
+            // the forward's centred ray rows (centred_rows), the raw transMat
+            // rows, the colour and the normal
             const float4 q0 = r[0], q1 = r[1], q2 = r[2], q3 = r[3], q4 = r[4];
             f3 R0, nAx, nAy;
             centred_rows({q0.x, q0.y, q0.z}, {q0.w, q1.x, q1.y}, {q1.z, q1.w, q2.x}, q2.y, q2.z, R0, nAx, nAy);
             s_r[wave][0][lane] = make_float4(R0.x, R0.y, R0.z, nAx.x);
             s_r[wave][1][lane] = make_float4(nAx.y, nAx.z, nAy.x, nAy.y);
             s_r[wave][2][lane] = make_float4(nAy.z, q2.y, q2.z, q2.w);
-            if constexpr (FULL) {
-                s_r[wave][3][lane] = q0;
-                s_r[wave][4][lane] = q1;
-                s_r[wave][5][lane] = make_float4(q2.x, q3.w, q4.x, q4.y);
-                s_r[wave][6][lane] = make_float4(q3.x, q3.y, q3.z, 0.f);
-            } else {
-                s_r[wave][3][lane] = make_float4(q3.w, q4.x, q4.y, 0.f);
-            }
-            if constexpr (FULL) L.e[wave][lane] = e;
+            s_r[wave][3][lane] = q0;
+            s_r[wave][4][lane] = q1;
+            s_r[wave][5][lane] = make_float4(q2.x, q3.w, q4.x, q4.y);
+            s_r[wave][6][lane] = make_float4(q3.x, q3.y, q3.z, 0.f);
+            s_e[wave][lane] = e;
         }
         wave_lds_sync();
-        // image-only: the entries' addresses are uniform (scalar loads),
-        // each fetched one visit ahead so its latency is not waited on, and
-        // an entry's ballot is the lane mask of `has` itself
-        uint4 e_next;
-        if constexpr (!FULL) e_next = lg[m - 1];
         for (int j = m - 1; j >= 0; --j) {
-            uint4 e;
-            if constexpr (FULL) {
-                e = L.e[wave][j];
-            } else {
-                e = e_next;
-                e_next = lg[max(j - 1, 0)];
-            }
-            const bool has = FULL ? (((lane < 32 ? e.x : e.y) >> (lane & 31)) & 1u)
-                                  : __builtin_amdgcn_inverse_ballot_w64(((uint64_t)e.y << 32) | e.x);
+            const uint4 e = s_e[wave][j];
+            const bool has = ((lane < 32 ? e.x : e.y) >> (lane & 31)) & 1u;
             float v16[16];
-            if constexpr (!FULL) {
-                const float4 q0 = s_r[wave][0][j], q1 = s_r[wave][1][j], q2 = s_r[wave][2][j];
-                const float4 q3 = s_r[wave][3][j];
-                const float opa = q2.w;
-                const float dxs = q2.y - px, dys = q2.z - py;
-                const float rx = __builtin_fmaf(dxs, q0.w, __builtin_fmaf(dys, q1.z, q0.x));
-                const float ry = __builtin_fmaf(dxs, q1.x, __builtin_fmaf(dys, q1.w, q0.y));
-                const float rz = __builtin_fmaf(dxs, q1.y, __builtin_fmaf(dys, q2.x, q0.z));
-                const float inv_z = has ? __builtin_amdgcn_rcpf(rz) : 0.f;
-                const float u = rx * inv_z, v = ry * inv_z;
-                const float rho3d = __builtin_fmaf(u, u, v * v);
-                const float rho2d = FILTER_INV_SQ * __builtin_fmaf(dxs, dxs, dys * dys);
-                const bool use3d = rho3d <= rho2d;
-                // zero where the lane did not blend: alpha, the transmittance
-                // factor, the suffix update and every gradient term follow
-                const float G =
-                    has ? __builtin_amdgcn_exp2f(__builtin_fminf(rho3d, rho2d) * -0.72134752044448170368f) : 0.f;
-                const float alpha = __builtin_fminf(0.99f, opa * G);
-                const float inv_om = __builtin_amdgcn_rcpf(1.0f - alpha);
-                Tr *= inv_om;  // transmittance before this splat (unchanged where it did not blend)
-                const float aT = alpha * Tr;
-                const float vv = __builtin_fmaf(dp0, q3.x, __builtin_fmaf(dp1, q3.y, dp2 * q3.z));  // dL/dimage . colour
-                // acc_v is the suffix behind this splat.  The reference
-                // folds a splat in when the next blended splat is reached
-                // (last_alpha / last_color, :1875-1876, :1919); folding it
-                // in as soon as it is done uses the same values, and
-                // alpha = 0 leaves the suffix unchanged without a select
-                const float dv = vv - acc_v;
-                const float dLda = __builtin_fmaf(dv, Tr, bgT * inv_om);
-                acc_v = __builtin_fmaf(alpha, dv, acc_v);
-                const float gg = dLda * G;
-                // dL/d(ray), up to the factor -opa, on the 3D branch: the
-                // ray-splat point (gg u, gg v) / ray.z pulled back through
-                // (u, v) = ray.xy / ray.z; its moments over the wave's pixels
-                // about the splat centre (sum dp, sum (xs - px) dp,
-                // sum (ys - py) dp) determine the nine transMat gradients
-                const float t = (use3d ? gg : 0.f) * inv_z;
-                const float dsx = t * u;
-                const float dsy = t * v;
-                const float dpz = -__builtin_fmaf(dsx, u, dsy * v);
-                // reduction slots (kImgRaw, kImgGrad): pairs (0, 8), (2, 10),
-                // (4, 12), (6, 14), (7, 15) and raw rows 1, 3, 5; the normal
-                // gradients (grads16 9-11) are zero here and take no slot
-                v16[0] = dsx;
-                v16[8] = dys * dpz;
-                v16[1] = dsy;
-                v16[2] = dpz;
-                v16[10] = dxs * dsx;
-                v16[3] = dxs * dsy;
-                v16[4] = dxs * dpz;
-                v16[12] = gg;
-                v16[5] = dys * dsx;
-                v16[6] = dys * dsy;
-                v16[14] = aT * dp1;
-                v16[7] = aT * dp0;
-                v16[15] = aT * dp2;
-                v16[9] = v16[11] = v16[13] = 0.f;  // raw rows' partners: not read
-            } else {
+            {
                 const float4 c0 = s_r[wave][0][j], c1 = s_r[wave][1][j], c2 = s_r[wave][2][j];
                 const float4 q0 = s_r[wave][3][j], q1 = s_r[wave][4][j], q5 = s_r[wave][5][j];
                 const float4 q6 = s_r[wave][6][j];
@@ -611,8 +779,8 @@ __global__ __launch_bounds__(kThreads) void k_raster_bwd(
                 v16[8] = px * dk.z + py * dl.z + dL_dz;
                 v16[12] = G * dL_dG * (1.0f - opa);
             }
-            const float s = FULL ? wave_reduce16(v16, lane) : wave_reduce16_lds8<kImgRaw>(v16, red8);
-            if (adds && s != 0.f) unsafeAtomicAdd(&grads16[(size_t)e.w * 16 + gi], s);
+            const float s = wave_reduce16(v16, lane);
+            if ((lane & 3) == 0 && s != 0.f) unsafeAtomicAdd(&grads16[(size_t)e.w * 16 + gi], s);
         }
         wave_lds_sync();
     }
@@ -1055,7 +1223,10 @@ void launch_check_rcp(hipStream_t s, int efield, unsigned long long *bad) {
     hipLaunchKernelGGL(k_check_rcp, dim3((1u << 24) / 256), dim3(256), 0, s, (uint32_t)efield, bad);
 }
 
-// Frames whose tiles leave most of the chip's wave slots empty.  FEW_MEASURED
+// Frames whose tiles leave most of the chip's wave slots empty: at most two
+// workgroups per CU, of the seven that fit.  294 tiles (324 x 210, 100k splats)
+// take 138 us on the small-frame kernel and 171 on the other; at 4346 tiles the
+// other keeps seven waves per SIMD busy, and this one would leave room for three.
 static bool few_tiles(int tiles_x, int tiles_y) { return (int64_t)tiles_x * tiles_y <= 512; }
 
 void launch_raster_fwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, const int *order, const int *offsets, const int *ids,
@@ -1135,18 +1306,22 @@ bool launch_raster_bwd(hipStream_t s, int W, int H, int tiles_x, int tiles_y, co
                        const float *dL_dmedian, const float *dL_ddist, float ddist_uniform, float *grads16,
                        const DeepTiles &deep) {
     const int grid = tile_order_ints(tiles_x, tiles_y);
-    const bool full = dL_ddepth || dL_daccum || dL_dnormal || dL_dmedian || dL_ddist || ddist_uniform != 0.0f;
+    const bool full = dL_ddepth || dL_daccum || dL_dnormal || dL_dmedian || dL_ddist;
+    const auto *rec4 = reinterpret_cast<const float4 *>(rec);
+    const bool few = few_tiles(tiles_x, tiles_y);
     auto launch = [&](hipStream_t st, int blocks, const int *list, int deep_len) {
+        const auto image = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, st, W, H, tiles_x, list, offsets, blog, rec4, bg,
+                               final_Ts, dL_dimg, ddist_uniform, grads16, deep_len);
+        };
         if (full)
-            hipLaunchKernelGGL(k_raster_bwd<true>, dim3(blocks), dim3(kThreads), 0, st, W, H, tiles_x, list, offsets, blog,
-                               reinterpret_cast<const float4 *>(rec), bg, final_Ts, final_idx,
-                               dL_dimg, dL_ddepth, dL_daccum, dL_dnormal, dL_dmedian, dL_ddist, ddist_uniform,
-                               grads16, deep_len);
+            hipLaunchKernelGGL(k_raster_bwd_full, dim3(blocks), dim3(kThreads), 0, st, W, H, tiles_x, list, offsets,
+                               blog, rec4, bg, final_Ts, final_idx, dL_dimg, dL_ddepth, dL_daccum, dL_dnormal,
+                               dL_dmedian, dL_ddist, ddist_uniform, grads16, deep_len);
+        else if (ddist_uniform != 0.0f)
+            image(few ? k_raster_bwd_few<true> : k_raster_bwd<true>);
         else
-            hipLaunchKernelGGL(k_raster_bwd<false>, dim3(blocks), dim3(kThreads), 0, st, W, H, tiles_x, list, offsets,
-                               blog, reinterpret_cast<const float4 *>(rec), bg, final_Ts, final_idx,
-                               dL_dimg, dL_ddepth, dL_daccum, dL_dnormal, dL_dmedian, dL_ddist, ddist_uniform,
-                               grads16, deep_len);
+            image(few ? k_raster_bwd_few<false> : k_raster_bwd<false>);
     };
     if (deep.n > 0) {
         // the deep tiles' long log replays start at once, on their own

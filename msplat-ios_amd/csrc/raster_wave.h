@@ -284,22 +284,25 @@ struct Red8 {
     }
 };
 
+// The reduction in two halves, so that several visits' rows can be written
+// before the first is read (each to its own scratch, `off` floats from r's).
 template <unsigned RAW, unsigned SKIP>
-__device__ __forceinline__ float wave_reduce16_lds8(float v[16], const Red8<RAW, SKIP> &r) {
+__device__ __forceinline__ void reduce16_write(float v[16], const Red8<RAW, SKIP> &r, int off = 0) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         if ((SKIP >> i) & 1u) continue;
         if ((RAW >> i) & 1u) {
-            r.wb[i & 3][64 * i] = v[i];
+            r.wb[i & 3][64 * i + off] = v[i];
             continue;
         }
         const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 8]), false,
                                                         false);
-        r.wb[i & 3][64 * i] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+        r.wb[i & 3][64 * i + off] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
     }
-    wave_lds_sync();
-    const float4 p = *r.r0, q = *r.r1;
-    wave_lds_sync();
+}
+template <unsigned RAW, unsigned SKIP>
+__device__ __forceinline__ float reduce16_read(const Red8<RAW, SKIP> &r, int off = 0) {
+    const float4 p = r.r0[off / 4], q = r.r1[off / 4];
     float s = ((p.x + p.y) + (p.z + p.w)) + ((q.x + q.y) + (q.z + q.w));
     s += dpp<kDppQuad1032>(s);
     s += dpp<kDppQuad2301>(s);
@@ -311,6 +314,14 @@ __device__ __forceinline__ float wave_reduce16_lds8(float v[16], const Red8<RAW,
         asm("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_shl:4 row_mask:%1 bank_mask:%2"
             : "+v"(s)
             : "n"(raw_dpp_rows(RAW)), "n"(raw_dpp_banks(RAW)));
+    return s;
+}
+template <unsigned RAW, unsigned SKIP>
+__device__ __forceinline__ float wave_reduce16_lds8(float v[16], const Red8<RAW, SKIP> &r) {
+    reduce16_write(v, r);
+    wave_lds_sync();
+    const float s = reduce16_read(r);
+    wave_lds_sync();
     return s;
 }
 
