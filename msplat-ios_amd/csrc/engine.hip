@@ -981,7 +981,8 @@ int msplat_hip_mc_table(int8_t tri[256 * 16]) {
 
 namespace {
 bool grid_args_ok(const float *grid, int dx, int dy, int dz, const float origin[3]) {
-    // (the TSDF launch needs its 8 x 8 x 4 bricks, padded to 8, in an int)
+    // (the TSDF launch needs its 8 x 8 x 8 bricks, padded to 8, in an int;
+    // checked for bricks of half that depth)
     if (!grid || !origin || dx < 1 || dy < 1 || dz < 1 || dz > 65535 ||
         (uint64_t)dx * (uint64_t)dy >= (uint64_t(1) << 32) ||
         (int64_t)((dx + 7) / 8) * ((dy + 7) / 8) * ((dz + 3) / 4) > (int64_t)INT_MAX - 8) {

@@ -109,7 +109,8 @@ __global__ __launch_bounds__(kThreads) void k_tsdf_blocks(const TsdfViewDev *__r
     if ((lane & (kTsdfBlock - 1)) == 0 && in) D.blk[band * D.blk_w + (px >> 4)] = m;
 }
 
-constexpr int kBrickX = 8, kBrickY = 8, kBrickZ = 4;
+constexpr int kBrickX = 8, kBrickY = 8, kBrickZ = 8;
+constexpr int kPerLane = kBrickZ / 4;  // voxels per thread, four slices apart
 // Eight lanes test one view against the brick, one corner each: a workgroup
 // tests 32 views at once.
 constexpr int kTestLanes = 8, kTestViews = kThreads / kTestLanes;
@@ -198,8 +199,9 @@ __device__ __forceinline__ float div_by(float x, float z, float r) {
     return __builtin_fmaf(__builtin_fmaf(-q, z, x), r, q);
 }
 
-// One thread per voxel; a workgroup owns an 8 x 8 x 4 brick and each wave a
-// 4 x 4 x 4 sub-brick, so a wave's voxels project to a compact patch of
+// A workgroup owns an 8 x 8 x 8 brick and each wave a 4 x 4 column of it, four
+// slices at a time (kPerLane voxels per thread, their loads in flight
+// together), so a wave's voxels project to a compact patch of
 // every view rather than a long image-space line, and bricks go to the
 // XCDs in contiguous bands (msd::xcd_tile), so neighbouring bricks, whose
 // patches overlap, share an L2.  32 views at a time are tested against the
@@ -207,11 +209,14 @@ __device__ __forceinline__ float div_by(float x, float z, float r) {
 // order with the reference kernel's update, reads the voxel on its first
 // update and writes it once at the end (untouched voxels are neither read
 // nor written, as in the reference).
-// Bound by the issue of the remaining pairs: two correctly rounded divisions
-// each, which share one reciprocal, and two dependent loads.  300^3 voxels of
-// 2 mm, 32 views of 1297 x 840 of a 0.2 m ball: 627 us, and 82 us for the
-// block maxima (3.4 TB/s); every pair evaluated, with a bit mask of the
-// passing pixels in place of the block maxima, took 2054 + 100 us.
+// Bound by the remaining pairs: two correctly rounded divisions each, which
+// share one reciprocal, and the cache lines of the maps (a wave's 64 pixels
+// lie on some 14 image rows), which are read only where the voxel's own block
+// can pass.  300^3 voxels of 2 mm, 32 views of 1297 x 840 of a 0.2 m ball:
+// 538 us, of which the brick tests are 133, and 82 us for the block maxima
+// (3.4 TB/s).  8 x 8 x 4 bricks without the voxels' block test took 627 us;
+// every pair evaluated, with a bit mask of the passing pixels in place of the
+// block maxima, 2054 + 100 us.
 __global__ __launch_bounds__(kThreads) void k_tsdf_integrate(float2 *__restrict__ grid, int nx, int ny, int nz,
                                                              int bx, int by, int nbricks, float ox, float oy,
                                                              float oz, float vs,
@@ -225,12 +230,18 @@ __global__ __launch_bounds__(kThreads) void k_tsdf_integrate(float2 *__restrict_
     const int x = b_x * kBrickX + (wave & 1) * 4 + (lane & 3);
     const int y = b_y * kBrickY + (wave >> 1) * 4 + ((lane >> 2) & 3);
     const int z = b_z * kBrickZ + (lane >> 4);
-    const bool in = x < nx && y < ny && z < nz;
-    const int64_t vid = ((int64_t)z * ny + y) * nx + x;
-    // voxel centre (msplat_metal.metal:2240-2243)
+    bool in[kPerLane];
+    int64_t vid[kPerLane];
+    // voxel centres (msplat_metal.metal:2240-2243)
     const float wx = ox + ((float)x + 0.5f) * vs;
     const float wy = oy + ((float)y + 0.5f) * vs;
-    const float wz = oz + ((float)z + 0.5f) * vs;
+    float wz[kPerLane];
+#pragma unroll
+    for (int q = 0; q < kPerLane; ++q) {
+        in[q] = x < nx && y < ny && z + 4 * q < nz;
+        vid[q] = ((int64_t)(z + 4 * q) * ny + y) * nx + x;
+        wz[q] = oz + ((float)(z + 4 * q) + 0.5f) * vs;
+    }
     // this lane's corner of the brick, its voxel centre by the same expression
     const int xc = min(b_x * kBrickX + (lane & 1) * (kBrickX - 1), nx - 1);
     const int yc = min(b_y * kBrickY + ((lane >> 1) & 1) * (kBrickY - 1), ny - 1);
@@ -238,8 +249,13 @@ __global__ __launch_bounds__(kThreads) void k_tsdf_integrate(float2 *__restrict_
     const float ccx = ox + ((float)xc + 0.5f) * vs;
     const float ccy = oy + ((float)yc + 0.5f) * vs;
     const float ccz = oz + ((float)zc + 0.5f) * vs;
-    float2 cur = make_float2(0.f, 0.f);
-    bool have = false;
+    float2 cur[kPerLane];
+    bool have[kPerLane];
+#pragma unroll
+    for (int q = 0; q < kPerLane; ++q) {
+        cur[q] = make_float2(0.f, 0.f);
+        have[q] = false;
+    }
     for (int k0 = 0, par = 0; k0 < nviews; k0 += kTestViews, par ^= 1) {
         const int kt = k0 + (int)threadIdx.x / kTestLanes;
         const bool may = view_may_update(views[min(kt, nviews - 1)], ccx, ccy, ccz, trunc) && kt < nviews;
@@ -258,42 +274,64 @@ __global__ __launch_bounds__(kThreads) void k_tsdf_integrate(float2 *__restrict_
         for (; todo; todo &= todo - 1u) {
             const TsdfViewDev &D = views[k0 + __builtin_ctz(todo)];
             const float *m = D.v.viewmat;
-            // world -> view (:2246-2249)
-            const float vx = m[0] * wx + m[1] * wy + m[2] * wz + m[3];
-            const float vy = m[4] * wx + m[5] * wy + m[6] * wz + m[7];
-            const float vz = m[8] * wx + m[9] * wy + m[10] * wz + m[11];
-            if (!in || vz <= 0.01f) continue;
-            // pinhole projection (:2252-2256)
-            const float r = msd::ms_rcp_nr(vz);
-            float tx = div_by(vx, vz, r), ty = div_by(vy, vz, r);
-            // outside the range of div_by (vz > 0.01 here)
-            if (!(__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(vx), __builtin_fabsf(vy)), vz) < 1e30f)) {
-                tx = vx / vz;
-                ty = vy / vz;
+            float vz[kPerLane], a[kPerLane], depth[kPerLane], dmax[kPerLane];
+            int64_t pid[kPerLane];
+            bool hit[kPerLane];
+#pragma unroll
+            for (int q = 0; q < kPerLane; ++q) {
+                // world -> view (:2246-2249)
+                const float vx = m[0] * wx + m[1] * wy + m[2] * wz[q] + m[3];
+                const float vy = m[4] * wx + m[5] * wy + m[6] * wz[q] + m[7];
+                vz[q] = m[8] * wx + m[9] * wy + m[10] * wz[q] + m[11];
+                // pinhole projection (:2252-2256)
+                const float r = msd::ms_rcp_nr(vz[q]);
+                float tx = div_by(vx, vz[q], r), ty = div_by(vy, vz[q], r);
+                hit[q] = in[q] && !(vz[q] <= 0.01f);
+                // outside the range of div_by (vz > 0.01 where it counts)
+                if (hit[q] && !(__builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(vx), __builtin_fabsf(vy)), vz[q]) < 1e30f)) {
+                    tx = vx / vz[q];
+                    ty = vy / vz[q];
+                }
+                const float px = tx * D.v.fx + D.v.cx;
+                const float py = ty * D.v.fy + D.v.cy;
+                const int ix = msd::f2i(px), iy = msd::f2i(py);
+                hit[q] = hit[q] && ix >= 0 && ix < D.v.width && iy >= 0 && iy < D.v.height;
+                pid[q] = (int64_t)iy * D.v.width + ix;
+                // the test of view_may_update for the voxel's own block: the
+                // wave's voxels share a few of those, where the maps' pixels
+                // lie on a cache line each or two
+                dmax[q] = hit[q] ? D.blk[(int64_t)(iy / kTsdfBlock) * D.blk_w + ix / kTsdfBlock] : 0.f;
             }
-            const float px = tx * D.v.fx + D.v.cx;
-            const float py = ty * D.v.fy + D.v.cy;
-            const int ix = msd::f2i(px), iy = msd::f2i(py);
-            if (ix < 0 || ix >= D.v.width || iy < 0 || iy >= D.v.height) continue;
-            const int64_t pid = (int64_t)iy * D.v.width + ix;
-            const float a = D.v.alpha_dev[pid];
-            const float depth = D.v.depth_dev[pid];
-            // the pixel tests (:2259-2265)
-            if (a < athr || !__builtin_isfinite(depth) || !(depth > 0.0f)) continue;
-            // truncated SDF and weighted running mean (:2267-2279)
-            float sdf = depth - vz;
-            if (sdf < -trunc) continue;
-            sdf = __builtin_fminf(__builtin_fmaxf(sdf, -trunc), trunc);
-            if (!have) {
-                cur = grid[vid];
-                have = true;
+#pragma unroll
+            for (int q = 0; q < kPerLane; ++q) {
+                hit[q] = dmax[q] > 0.f && !(dmax[q] - vz[q] < -trunc);
+                a[q] = depth[q] = 0.f;
+                if (hit[q]) {
+                    a[q] = D.v.alpha_dev[pid[q]];
+                    depth[q] = D.v.depth_dev[pid[q]];
+                }
             }
-            const float nw = cur.y + a;
-            cur.x = (cur.x * cur.y + sdf * a) / nw;
-            cur.y = nw;
+#pragma unroll
+            for (int q = 0; q < kPerLane; ++q) {
+                // the pixel tests (:2259-2265)
+                if (!hit[q] || a[q] < athr || !__builtin_isfinite(depth[q]) || !(depth[q] > 0.0f)) continue;
+                // truncated SDF and weighted running mean (:2267-2279)
+                float sdf = depth[q] - vz[q];
+                if (sdf < -trunc) continue;
+                sdf = __builtin_fminf(__builtin_fmaxf(sdf, -trunc), trunc);
+                if (!have[q]) {
+                    cur[q] = grid[vid[q]];
+                    have[q] = true;
+                }
+                const float nw = cur[q].y + a[q];
+                cur[q].x = (cur[q].x * cur[q].y + sdf * a[q]) / nw;
+                cur[q].y = nw;
+            }
         }
     }
-    if (have) grid[vid] = cur;
+#pragma unroll
+    for (int q = 0; q < kPerLane; ++q)
+        if (have[q]) grid[vid[q]] = cur[q];
 }
 
 // ---- marching cubes -----------------------------------------------------
@@ -327,15 +365,28 @@ __global__ __launch_bounds__(kThreads) void k_mc_classify(const float2 *__restri
     const int64_t nxy = (int64_t)nx * ny;
     const int cx = nx - 1, cy = ny - 1;
     uint32_t tris = 0;
+    // the cell's coordinates, divided once and advanced by kThreads cells
+    const int dj = kThreads / cx, di = kThreads - dj * cx;
+    const int64_t c0 = chunk * kMeshChunk + threadIdx.x;
+    int i = (int)(c0 % cx);
+    int64_t rest = c0 / cx;
+    int j = (int)(rest % cy), k = (int)(rest / cy);
     for (int r = 0; r < kPerThread; ++r) {
-        const int64_t c = chunk * kMeshChunk + r * kThreads + threadIdx.x;
+        const int64_t c = c0 + r * kThreads;
         uint32_t m = 0;
         if (c < ncells) {
-            const int i = (int)(c % cx);
-            const int64_t q = c / cx;
-            const int j = (int)(q % cy), k = (int)(q / cy);
             m = cell_case(grid, ((int64_t)k * ny + j) * nx + i, nx, nxy);
             tris += c_mc.ntri[m];
+        }
+        i += di;
+        j += dj;
+        if (i >= cx) {
+            i -= cx;
+            ++j;
+        }
+        while (j >= cy) {
+            j -= cy;
+            ++k;
         }
         cases[c] = (uint8_t)m;  // the case buffer covers whole chunks
     }
