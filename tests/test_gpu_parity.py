@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 from msplat import _engine as E  # noqa: E402
 from msplat import device as D  # noqa: E402
 from msplat import synthetic as S  # noqa: E402
-from parity import grad_close, param_grad_noise, post_adam_close  # noqa: E402
+from parity import RTOL, grad_close, param_grad_noise, post_adam_close  # noqa: E402
 from scenes import adversarial  # noqa: E402
 
 
@@ -515,3 +515,44 @@ def test_densify_split_and_dup_beyond_3n(orc, eng):
     for i, (d, o) in enumerate(zip(dev, params + m6 + v6)):
         st = strides[i % 6]
         _assert_bitexact(d.numpy()[: new_o * st], o[: new_o * st], f"buffer {i}")
+
+
+# 32 x 16 = 512 tiles is the last frame of the few-tile raster kernels and
+# 27 x 19 = 513 the first of the others; the ragged frames end inside a tile
+# in both directions, and 17 x 3 pixels are two tiles.
+@pytest.mark.parametrize("ldist", [0.0, 0.5], ids=["image", "distortion"])
+@pytest.mark.parametrize("W,H", [(17, 3), (512, 256), (505, 243), (432, 304), (419, 297)])
+def test_raster_kernels_around_the_few_tile_line(W, H, ldist, orc, eng):
+    """The forward bit for bit, and the training step's raster gradients
+    (unfused: its parameter gradients; fused: the first Adam moments) within
+    the summation bounds, with and without the distortion term."""
+    scene = S.make_scene(2, n=6000, width=W, height=H, num_cameras=2)
+    print(f"[few-tile line] {W}x{H} lambda_dist={ldist}", flush=True)
+    ocam, proj, bins, fwd, ds, gcam, out = _forward_both(scene, 0, orc, eng)
+    for k in ("out_img", "final_Ts", "final_idx", "out_depth", "out_normal", "out_alpha", "out_median_depth",
+              "out_distortion"):
+        _assert_bitexact(out[k], fwd[k], k)
+    gt = orc.render(scene.jittered(0.01, 99), 0)[3]["out_img"]
+    loss_o, dL, dreg, _ = orc.loss_fwd_bwd(fwd["out_img"], gt, distortion=fwd["out_distortion"], lambda_dist=ldist)
+    g_o, a_o = orc.raster_bwd(proj, bins, fwd, ocam, scene.background, dL, dL_ddist=dreg if ldist else None,
+                              with_abs=True)
+    assert np.abs(g_o).max() > 0
+    noise = param_grad_noise(orc, _params(scene), ocam, scene.sh_degree, scene.sh_degree, proj["radii"], g_o, a_o)
+    zeros = dict(grad_norm=np.zeros(scene.n, np.float32), vis=np.zeros(scene.n, np.float32),
+                 max2d=np.zeros(scene.n, np.float32))
+    po = orc.project_bwd(_params(scene), ocam, scene.sh_degree, scene.sh_degree, proj["radii"], g_o, zeros)
+    want = [po["dmeans"], po["dscales"], po["dquats"], po["dfdc"], po["dfrest"], g_o[:, 12]]
+    d_gt = _device(gt)
+    for fused in (False, True):
+        ds = D.DeviceScene(scene)
+        loss, nis = D.train_step(ds, gcam, d_gt, fused_adam=fused, lambda_dist=ldist)
+        assert nis == bins["ids"].size
+        assert abs(loss - loss_o) <= 1e-5 * abs(loss_o) + 1e-9
+        grad_close(E.last("grads16", (scene.n, 16)), g_o, a_o, f"grads16 {W}x{H} lambda_dist={ldist} fused={fused}")
+        for m, w, nz in zip(ds.exp_avg, want, noise):
+            g = m.numpy().astype(np.float64).reshape(-1) / (1.0 - 0.9)
+            w = np.asarray(w, np.float64).reshape(-1)
+            # the bound of post_adam_close: the propagated raster bound, plus
+            # the relative terms of the summation and of the moment itself
+            allowed = nz + (RTOL + 2.5e-7) * np.abs(w) + 1e-30
+            assert (np.abs(g - w) <= allowed).all()
