@@ -1396,17 +1396,18 @@ static int densify_impl(int scale_dim, int n, int capacity, float grad_thresh, f
     if (E.dens_flags.cap < (size_t)n * 16)
         CHECK(ensure(E.dens_flags, (size_t)std::min<int64_t>(2 * (int64_t)n, capacity) * 16));
     // the count after appending is at most 4N (a splat can be split and dup)
-    CHECK(ensure(E.dens_scan, (size_t)mskern::scan_temp_ints(4 * (int64_t)n) * 4));
+    CHECK(ensure(E.dens_scan, (size_t)mskern::densify_scan_ints(n) * 4));
     int *f = P<int>(E.dens_flags);
     a.split = f;
     a.dup = f + n;
     a.split_pre = f + 2 * (size_t)n;
     a.dup_pre = f + 3 * (size_t)n;
     a.scan_temp = P<int>(E.dens_scan);
-    mskern::launch_densify_classify(E.stream, a);
+    const int *n_split, *n_dup;
+    mskern::launch_densify_classify(E.stream, a, n_split, n_dup);
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(E.pinned_i, a.split_pre + n - 1, sizeof(int), hipMemcpyDeviceToHost, E.stream));
-    HIPC(hipMemcpyAsync(E.pinned_i + 1, a.dup_pre + n - 1, sizeof(int), hipMemcpyDeviceToHost, E.stream));
+    HIPC(hipMemcpyAsync(E.pinned_i, n_split, sizeof(int), hipMemcpyDeviceToHost, E.stream));
+    HIPC(hipMemcpyAsync(E.pinned_i + 1, n_dup, sizeof(int), hipMemcpyDeviceToHost, E.stream));
     HIPC(hipStreamSynchronize(E.stream));
     // A splat that is small but wide on screen is classified both split and
     // dup (msplat_metal.metal:3250-3262), so the appended count can exceed
@@ -1440,9 +1441,9 @@ static int densify_impl(int scale_dim, int n, int capacity, float grad_thresh, f
     a.keep_pre = a.keep + n_new;
     a.src_of = a.keep + 2 * n_new;
     a.parent = a.keep + 3 * n_new;
-    mskern::launch_densify_apply(E.stream, a, E.pinned_i[0], (int)n_new);
+    const int *count = mskern::launch_densify_apply(E.stream, a, E.pinned_i[0], (int)n_new);
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(E.pinned_i, a.keep_pre + n_new - 1, sizeof(int), hipMemcpyDeviceToHost, E.stream));
+    HIPC(hipMemcpyAsync(E.pinned_i, count, sizeof(int), hipMemcpyDeviceToHost, E.stream));
     HIPC(hipStreamSynchronize(E.stream));
     *new_count = E.pinned_i[0];
     return MSPLAT_OK;

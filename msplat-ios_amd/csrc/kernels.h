@@ -200,8 +200,6 @@ void launch_zero_counters(hipStream_t s, int *a, int na, int *b, int nb);
 // Publishes the two loss doubles and the n_ctr counters (data: two doubles,
 // then the counters) behind everything queued on s.
 void launch_step_report(hipStream_t s, const double *loss, const int *ctr, int n_ctr, const Publish &out);
-int64_t scan_temp_ints(int64_t n);
-void launch_scan_i32(hipStream_t s, const int *in, int *out, int n, int *temp);
 
 struct DensifyArgs {
     int n, fr_stride;
@@ -215,19 +213,23 @@ struct DensifyArgs {
     float *params[6], *exp_avg[6], *exp_avg_sq[6];
     float *workspace;  // densify_workspace_floats(n_virt, scale_dim, fr_stride) floats
     const float *random;
-    int *split, *dup, *split_pre, *dup_pre, *scan_temp;
+    int *split, *dup;             // n flags each
+    int *split_pre, *dup_pre;     // their prefixes inside each scan tile
+    int *scan_temp;               // densify_scan_ints(n) ints
     int *keep, *keep_pre, *src_of;  // n_virt entries each
     int *parent;                    // n_virt - n entries
 };
-// Classification and the split / dup prefix counts (the count after
-// appending is N + 2 * split_pre[N-1] + dup_pre[N-1]; a splat can be both).
-void launch_densify_classify(hipStream_t s, const DensifyArgs &a);
+// Classification and the split / dup counts, left at n_split and n_dup
+// (device; the count after appending is N + 2 nS + nD; a splat can be both).
+int64_t densify_scan_ints(int64_t n);
+void launch_densify_classify(hipStream_t s, const DensifyArgs &a, const int *&n_split, const int *&n_dup);
 // Keep flags of the old and appended rows, the gather of every surviving
-// row into the workspace and its copy back into the caller's buffers.
-// n_virt = n + 2 nS + nD (the count after appending) must fit the buffers'
-// capacity; the new count is keep_pre[n_virt - 1].  Strides up to 127.
+// row (output rows from n on in place, the others into the workspace) and
+// the staged rows' copy into the caller's buffers.  n_virt = n + 2 nS + nD
+// (the count after appending) must fit the buffers' capacity; returns where
+// the new count is (device).  Strides up to 127.
 int64_t densify_workspace_floats(int n_virt, int scale_dim, int fr_stride);
-void launch_densify_apply(hipStream_t s, const DensifyArgs &a, int nS, int n_virt);
+const int *launch_densify_apply(hipStream_t s, const DensifyArgs &a, int nS, int n_virt);
 
 // k_mesh.hip
 // The compaction passes work on chunks of kMeshChunk cells / pixels: one

@@ -556,3 +556,39 @@ def test_raster_kernels_around_the_few_tile_line(W, H, ldist, orc, eng):
             # the relative terms of the summation and of the moment itself
             allowed = nz + (RTOL + 2.5e-7) * np.abs(w) + 1e-30
             assert (np.abs(g - w) <= allowed).all()
+
+
+# The scans' tiles hold 1024 splats and the gather's blocks 256 rows; "grow"
+# ends above N (output rows from N on are written in place), "shrink" below
+# it (every row is staged), "swap" close to N.
+@pytest.mark.parametrize("kind", ["grow", "shrink", "swap"])
+@pytest.mark.parametrize("n", [1, 255, 257, 1024, 1025, 4099])
+def test_densify_at_the_tile_edges(n, kind, orc, eng):
+    scene = S.make_scene(5, n=n, width=320, height=208, num_cameras=1)
+    scene.scales[::3] += np.float32(2.0)
+    scene.opacities[:: {"grow": 11, "shrink": 1, "swap": 2}[kind]] = np.float32(-6.0)
+    if kind == "shrink":
+        scene.opacities[::5] = np.float32(1.0)
+    cap = 4 * n + 3
+    params, m6, v6, strides, stats, rs = _densify_inputs(scene, n, cap, 100 + n)
+    print(f"[densify] n={n} {kind}", flush=True)
+    dev = [_device(a) for a in params + m6 + v6]
+    dstats = {k: _device(v) for k, v in stats.items()}
+    d_rs = _device(rs)
+    P6 = C.c_void_p * 6
+    newc = C.c_int()
+    E.check(E.lib().msplat_hip_densify(n, cap, 0.0002, 0.01, 0.05, 1, 0.1, 0.5, 0.15, 0, dstats["grad_norm"].ptr,
+                                       dstats["vis"].ptr, dstats["max2d"].ptr, 648.5,
+                                       P6(*[d.ptr for d in dev[0:6]]), strides[4], P6(*[d.ptr for d in dev[6:12]]),
+                                       P6(*[d.ptr for d in dev[12:18]]), d_rs.ptr, C.byref(newc)))
+    new_o = orc.densify(n, cap, params, m6, v6, strides[4], stats, rs, 0.0002, 0.01, 0.05, 1, 0.1, 0.5, 0.15, 0,
+                        half_max_dim=648.5)
+    assert newc.value == new_o
+    if n > 1:
+        assert {"grow": new_o > n, "shrink": new_o < n, "swap": new_o != n}[kind], (n, new_o)
+    for i, (d, o) in enumerate(zip(dev, params + m6 + v6)):
+        s = strides[i % 6]
+        got = d.numpy()
+        _assert_bitexact(got[: new_o * s], o[: new_o * s], f"buffer {i}")
+        # nothing is written past the rows there are or were
+        assert not got[max(n, new_o) * s:].any()
