@@ -648,11 +648,11 @@ struct TileCounts {
 };
 
 // Counts the entries of the super-tile's 16 tiles into tile_counts, then
-// sorts the super-tile list in place, for lists of above and up to CAP keys
-// (the others belong to another launch).  With CAP = kRun longer lists are
-// queued on huge_list (their tile counts zeroed): k_sort_runs sorts their
-// runs on many workgroups, and after the merge passes k_count_chunks /
-// k_emit_chunks count and emit them chunk by chunk.
+// sorts the super-tile list in place, for lists of above and up to CAP keys.
+// Longer lists belong to another launch, or are queued on huge_list when
+// there is one (their tile counts zeroed): k_sort_runs sorts their runs on
+// many workgroups, and after the merge passes k_count_chunks / k_emit_chunks
+// count and emit them chunk by chunk.
 template <bool PACKED, int CAP, int THREADS>
 __global__ __launch_bounds__(THREADS) void k_sort_super(int tiles_x, int tiles_y, int sxn,
                                                         const int *__restrict__ offsets,
@@ -664,7 +664,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_super(int tiles_x, int tiles_y
     __shared__ typename Sort::Lds L;
     const int t = blockIdx.x;
     const int start = offsets[t], cnt = offsets[t + 1] - start;
-    if (cnt <= above || (CAP < kRun && cnt > CAP)) return;
+    if (cnt <= above || (!huge_list && cnt > CAP)) return;
     const int stx = (t % sxn) * kSuper, sty = (t / sxn) * kSuper;
     Sort st;
     if (threadIdx.x < kTiles) L.tc[threadIdx.x] = 0;
@@ -1000,7 +1000,12 @@ __device__ __forceinline__ void emit_range(const unsigned long long *__restrict_
 // workgroup per XCD.  With the blob scene of 500k splats at 1297 x 840 the
 // render forward takes 205 us instead of 228, at 200k splats the full-output
 // forward 229 instead of 254; 3M splats at 5187 x 3361 2410 instead of 2466.
-constexpr int kLenClasses = 16;
+// A class spans at least 32 entries: lists that differ by less take the same
+// time, and neighbours kept together complete each other's cache lines of the
+// output (6k splats at 3262 x 2165, a list or two per tile: image and full
+// outputs 302 us with classes of one entry and blocks of 4 x 4 tiles, 268 with
+// these and 8 x 8).
+constexpr int kLenClasses = 16, kMinLenClass = 32;
 __device__ __forceinline__ void order_tiles(int x, int tiles_x, int tiles_y, int quarter,
                                             const int *__restrict__ toffsets, int *s_n, int *__restrict__ order) {
     const int slots = msd::xcd_strip_grid(tiles_x, tiles_y) / 8;
@@ -1030,7 +1035,7 @@ __device__ __forceinline__ void order_tiles(int x, int tiles_x, int tiles_y, int
     }
 }
 
-// Emits each super-tile list of at most kRun entries into its 16 tile lists
+// Emits each super-tile list of at most `most` entries into its 16 tile lists
 // (longer lists: k_emit_chunks).  The first eight workgroups order the tiles
 // for the rasterizers (order_tiles) meanwhile.
 template <bool PACKED>
@@ -1039,7 +1044,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_tiles(int tiles_x, int ti
                                                              const unsigned long long *__restrict__ skeys,
                                                              const uint2 *__restrict__ rect,
                                                              const int *__restrict__ toffsets,
-                                                             int *__restrict__ ids, int tiles_quarter,
+                                                             int *__restrict__ ids, int most, int tiles_quarter,
                                                              int *__restrict__ order) {
     __shared__ EmitLds L;
     if (blockIdx.x < 8) {
@@ -1049,7 +1054,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_emit_tiles(int tiles_x, int ti
     const int st = blockIdx.x - 8;
     const int stx = (st % sxn) * kSuper, sty = (st / sxn) * kSuper;
     const int start = soffsets[st], cnt = soffsets[st + 1] - start;
-    if (cnt > kRun) return;
+    if (cnt > most) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tx = stx + wave % kSuper, ty = sty + wave / kSuper;
     const int out = (tx < tiles_x && ty < tiles_y) ? toffsets[ty * tiles_x + tx] : -1;
@@ -1163,12 +1168,18 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
     // 4096 keys go first, on the small sort, and the larger one takes the
     // rest (its other workgroups end at once): 4346 lists 87 + 22 us against
     // 200 us all on the middle sort.
-    const auto sort = [&](auto kernel, int threads, int above) {
+    // Where the frame has huge lists, which are sorted and emitted on many
+    // workgroups, those above 8192 keys join them, instead of one workgroup
+    // each on the largest sort and in the emission: frame of 500k splats at
+    // 375 x 378 443 -> 411 us, step of 767k at 334 x 297 675 -> 626.
+    const bool huge = super_max > kRun;
+    const int most = huge ? 8192 : kRun;
+    const auto sort = [&](auto kernel, int threads, int above, bool queue = false) {
         hipLaunchKernelGGL(kernel, dim3(NS), dim3(threads), 0, s, tiles_x, tiles_y, sxn, super_offsets, k, r2,
-                           tile_counts, huge_list, huge_stats, above);
+                           tile_counts, queue ? huge_list : nullptr, huge_stats, above);
     };
     constexpr int kCus = 256;
-    const bool mid = super_max <= 8192;
+    const bool mid = huge || super_max <= 8192;
     int above = -1;
     if (super_max <= 4096 || NS > (mid ? 2 * kCus : kCus)) {
         sort(packed ? k_sort_super<true, 4096, 512> : k_sort_super<false, 4096, 512>, 512, above);
@@ -1176,7 +1187,7 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
     }
     if (super_max > 4096) {
         if (mid)
-            sort(packed ? k_sort_super<true, 8192, 1024> : k_sort_super<false, 8192, 1024>, 1024, above);
+            sort(packed ? k_sort_super<true, 8192, 1024> : k_sort_super<false, 8192, 1024>, 1024, above, huge);
         else
             sort(packed ? k_sort_super<true, kRun, 1024> : k_sort_super<false, kRun, 1024>, 1024, above);
     }
@@ -1184,7 +1195,6 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
     // chunk and merge-tile kernels stride over units numbered across all
     // their lists; their grids cover at most total_keys / unit + NS units
     // (each list rounds up once)
-    const bool huge = super_max > kRun;
     const int huge_grid = (int)std::min<int64_t>(4096, (int64_t)total_keys / kChunk + NS);
     if (huge) {
         const UnitList chunks{huge_list, huge_stats, kChunk, chunk_base, huge_stats + 1};
@@ -1214,8 +1224,8 @@ void launch_bin_tiles(hipStream_t s, int n, int tiles_x, int tiles_y, const int 
     }
     launch_scan_counts(s, T, tile_counts, tile_offsets, tile_stats, tile_temp, x);
     hipLaunchKernelGGL(packed ? k_emit_tiles<true> : k_emit_tiles<false>, dim3(8 + NS), dim3(kEmitThreads), 0, s,
-                       tiles_x, tiles_y, sxn, super_offsets, k, r2, tile_offsets, ids,
-                       std::max(1, num_isect / (4 * T)), tile_order);
+                       tiles_x, tiles_y, sxn, super_offsets, k, r2, tile_offsets, ids, most,
+                       std::max(kMinLenClass, num_isect / (4 * T)), tile_order);
     if (huge)
         hipLaunchKernelGGL(packed ? k_emit_chunks<true> : k_emit_chunks<false>, dim3(huge_grid), dim3(kEmitThreads), 0,
                            s, tiles_x, tiles_y, sxn, super_offsets, huge_list, huge_stats, chunk_base, chunk_counts, k,

@@ -101,8 +101,9 @@ constexpr int kSuperTile = 4;
 // Keys of a super-tile list that one workgroup sorts in LDS, and keys per
 // counting and emission unit of a longer (huge) list.
 constexpr int kSuperSortRun = 16384, kSuperChunk = 4096;
-// Whether some list exceeds kSuperSortRun: those lists are sorted in runs,
-// merged, counted and emitted by many workgroups each.
+// Whether some list exceeds kSuperSortRun: those lists, and with them the
+// ones above half of it, are sorted in runs, merged, counted and emitted by
+// many workgroups each.
 inline bool bin_huge_lists(int super_max) { return super_max > kSuperSortRun; }
 // Ints of chunk_counts: 16 per chunk of the huge lists, at most
 // total / kSuperChunk + NS chunks.

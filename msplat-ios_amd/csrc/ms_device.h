@@ -712,7 +712,9 @@ __device__ __forceinline__ int xcd_tile(int block, int num_tiles) {
 // dealt in turn, the columns rotated by three from one row of blocks to the
 // next (a row of 8 m blocks would otherwise give every XCD whole columns);
 // inside a block a workgroup's neighbours share splats, whose records the
-// XCD's L2 then serves.  Larger pictures take larger blocks.  Returns the
+// XCD's L2 then serves.  Larger pictures take larger blocks, as soon as the
+// XCDs' shares stay even: a block's rows are the whole cache lines of the
+// outputs that one XCD writes.  Returns the
 // tile of workgroup `block`, or -1 for the padding of a grid of
 // xcd_strip_grid(tx, ty) workgroups.  A bijection onto [0, tx * ty).
 // Against bands of tile rows walked in strips of 8 (blob scenes): render
@@ -720,7 +722,7 @@ __device__ __forceinline__ int xcd_tile(int block, int num_tiles) {
 // 5187 x 3361 8.37 -> 8.25 ms.
 __host__ __device__ __forceinline__ int xcd_block_log2(int tx, int ty) {
     const long long t = (long long)tx * ty;
-    return t >= 32768 ? 3 : t >= 2048 ? 2 : 1;
+    return t >= 16384 ? 3 : t >= 2048 ? 2 : 1;
 }
 __host__ __device__ __forceinline__ int xcd_strip_grid(int tx, int ty) {
     const int l = xcd_block_log2(tx, ty), S = 1 << l;

@@ -592,3 +592,36 @@ def test_densify_at_the_tile_edges(n, kind, orc, eng):
         _assert_bitexact(got[: new_o * s], o[: new_o * s], f"buffer {i}")
         # nothing is written past the rows there are or were
         assert not got[max(n, new_o) * s:].any()
+
+
+@pytest.mark.parametrize("wide", [False, True], ids=["packed-keys", "wide-keys"])
+def test_middle_lists_join_the_huge_ones(wide, orc, eng):
+    """Super-tile lists of all sizes in a frame with one above 16384 keys:
+    those above 8192 take the run, count and emission chunks with it, the
+    shorter ones the in-LDS sorts."""
+    scene = _four_super_tiles()
+    E.check(E.lib().msplat_hip_set_wide_keys(1 if wide else 0))
+    try:
+        ocam, proj, bins, fwd, ds, gcam, out = _forward_both(scene, 0, orc, eng)
+    finally:
+        E.check(E.lib().msplat_hip_set_wide_keys(0))
+    offs, ids = bins["tile_offsets"], bins["ids"]
+    per = [np.unique(np.concatenate([ids[offs[y * 16 + x]:offs[y * 16 + x + 1]] for y in range(4)
+                                     for x in range(4 * s, 4 * s + 4)])).size for s in range(4)]
+    print(f"[middle lists] wide={wide} super-tile lists {per}", flush=True)
+    assert max(per) > 16384 and any(8192 < k <= 16384 for k in per) and any(0 < k <= 8192 for k in per), per
+    _assert_bitexact(E.last("tile_offsets"), bins["tile_offsets"], "tile offsets")
+    _assert_bitexact(E.last("gaussian_ids"), bins["ids"], "per-tile sorted ids")
+
+
+def _four_super_tiles():
+    counts = (18_000, 11_000, 6_000, 2_000)
+    scene = S.make_scene(1, n=sum(counts), width=256, height=64, seed=3)
+    rng = np.random.default_rng(3)
+    col = np.repeat(np.arange(4), counts)
+    fx = scene.cameras[0].fx
+    z = rng.uniform(-0.5, 0.5, col.size)
+    x = ((col + rng.uniform(0.2, 0.8, col.size)) * 64 - 128) / fx * 3.0
+    scene.means[:] = np.stack([x, rng.uniform(-20, 20, col.size) / fx * 3.0, z], 1).astype(np.float32)
+    scene.scales[:] = np.float32(np.log(2.0 / fx))
+    return scene
