@@ -163,7 +163,7 @@ def _depths(pattern, n, rng):
 
 @pytest.mark.parametrize("pattern,wide", [("even", False), ("plane", False), ("slab", False), ("planes", False),
                                           ("piled", False), ("even", True), ("slab", True)])
-@pytest.mark.parametrize("n", [1, 2, 65, 4096, 4097, 8192, 8193, 16384, 16385])
+@pytest.mark.parametrize("n", [1, 2, 3, 64, 65, 4096, 4097, 8192, 8193, 16384, 16385])
 def test_super_tile_sort_bitexact(n, pattern, wide, orc, eng):
     """One super-tile (64 x 64 pixels) whose list has n keys, around the
     capacities of the in-LDS sorts (4096, 8192, 16384 keys) and with depths
